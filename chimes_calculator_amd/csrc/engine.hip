@@ -2004,6 +2004,7 @@ struct chx_lmp {
     std::vector<double> out_h;
     DevBuf<double> x, out;
     DevBuf<int> ctype, tag, ilist, nbr_off, nbr, cnt, trips, quads, status, fp_cnt;
+    DevBuf<int> near;  // listed clusters within the cutoffs this step
     DevBuf<long long> off, fp_off;
     DevBuf<double> fp_rows;
     std::vector<int> fp_cnt_h;
@@ -2343,10 +2344,14 @@ int chx_lmp_compute(chx_lmp *p, int nall, const double *x, const int *type, cons
         launch_lmp_pair(A, m->dev, &p->tabs, st);
         HIPCHK(hipGetLastError());
         HIPCHK(hipEventRecord(p->ev[3], st));
+        // one scratch list: the triplets' is consumed before the quadruplets' is written (one stream)
+        if (p->n3 + p->n4 > 0) p->near.ensure((size_t)std::max(p->n3, p->n4));
         if (m->d.order[1] > 0 && p->n3 > 0)
-            launch_lmp_clusters(3, m->d.D3, p->n3, p->trips.p, A, m->dev, &p->tabs, st);
+            launch_lmp_clusters(3, m->d.D3, p->n3, p->trips.p, m->rc[1], p->near.p, p->status.p + CHX_LMP_ST_NEAR3, A,
+                                m->dev, &p->tabs, st);
         if (m->d.order[2] > 0 && p->n4 > 0)
-            launch_lmp_clusters(4, m->d.D4, p->n4, p->quads.p, A, m->dev, &p->tabs, st);
+            launch_lmp_clusters(4, m->d.D4, p->n4, p->quads.p, m->rc[2], p->near.p, p->status.p + CHX_LMP_ST_NEAR4, A,
+                                m->dev, &p->tabs, st);
         HIPCHK(hipGetLastError());
         const size_t nout = (size_t)nall * 3 + (nE ? nall : 0) + (nV ? (size_t)nall * 6 : 0) + 7;
         p->out.ensure(nout + CHX_LMP_ST_WORDS);

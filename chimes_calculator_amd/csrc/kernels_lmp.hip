@@ -292,93 +292,179 @@ __device__ __forceinline__ void tab3_cluster(const chx_model_dev &M, const chx_t
     }
 }
 
+// ---------------------------------------------------------------------------
+// The listed clusters that may be evaluated this step: every pair distance
+// within the largest cutoff of the body order.  The lists reach one skin
+// further, so most of their entries are outside (97% of the quadruplets and
+// 85% of the triplets of a 3.2 g/cc carbon box at 3.125 / 4 A with a 1.5 A
+// skin); evaluated one entry per lane, nearly every wavefront paid for the
+// whole polynomial with a few lanes active.  The test is on squared lengths
+// with a relative margin of 2^-40 on the limit (lim2), far above the rounding
+// of either form, so every cluster the exact test of the evaluation accepts
+// is kept.  Each workgroup takes NEAR_SPAN consecutive entries and appends its
+// survivors' list indices as one run, so neighbouring clusters stay together
+// for the force table; every sum is exact, so their order decides nothing.
+// Bound by the gathers of the members' positions (L2).
+// ---------------------------------------------------------------------------
+constexpr int NEAR_SPAN = 2048;
+
+template <int NB>
+__global__ __launch_bounds__(256) void k_lmp_near(long n, const int *__restrict__ list,
+                                                  const double *__restrict__ x, double lim2, int *near, int *count)
+{
+    constexpr int PER = NEAR_SPAN / 256;
+    __shared__ int wtot[PER][4];
+    __shared__ int base_s;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const long b0 = (long)blockIdx.x * NEAR_SPAN;
+    unsigned long long bal[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+        const long c = b0 + u * 256 + threadIdx.x;
+        bool in = false;
+        if (c < n) {
+            int m[NB];
+            if constexpr (NB == 4) {
+                const int4 q = reinterpret_cast<const int4 *>(list)[c];
+                m[0] = q.x; m[1] = q.y; m[2] = q.z; m[3] = q.w;
+            } else {
+#pragma unroll
+                for (int a = 0; a < NB; a++) m[a] = list[c * NB + a];
+            }
+            double p[NB][3];
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int k = 0; k < 3; k++) p[a][k] = x[3L * m[a] + k];
+            in = true;
+#pragma unroll
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = a + 1; b < NB; b++) {
+                    const double d0 = p[b][0] - p[a][0], d1 = p[b][1] - p[a][1], d2 = p[b][2] - p[a][2];
+                    in = in && d0 * d0 + d1 * d1 + d2 * d2 < lim2;
+                }
+        }
+        bal[u] = __ballot(in);
+        if (lane == 0) wtot[u][wv] = __popcll(bal[u]);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int t = 0;
+#pragma unroll
+        for (int u = 0; u < PER; u++)
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const int v = wtot[u][w];
+                wtot[u][w] = t;
+                t += v;
+            }
+        base_s = t ? atomicAdd(count, t) : 0;
+    }
+    __syncthreads();
+    const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+        if ((bal[u] >> lane) & 1)
+            near[base_s + wtot[u][wv] + __popcll(bal[u] & below)] = (int)(b0 + u * 256 + threadIdx.x);
+}
+
+// One thread per cluster of near[0 .. *count) (k_lmp_near); a fixed grid walks
+// them 128 at a time, since the host does not know their number.  4096 carbon
+// atoms at 3.2 g/cc, orders 5 / 3: one entry per lane over the whole lists took
+// 269 us (triplets) and 890 us (quadruplets), and a step of the pair style
+// 1426 us; selection and evaluation together leave a step of 504 us.
 template <int NB, int D, bool TAB>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k_lmp_clusters(long n, const int *__restrict__ list, chx_lmp_args A,
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k_lmp_clusters(const int *__restrict__ count, const int *__restrict__ near, const int *__restrict__ list, chx_lmp_args A,
                                                       chx_model_dev M, chx_tabs_dev T)
 {
     // the members' forces of the workgroup's clusters, merged per atom
     __shared__ fx_table<512> tab;  // >= 128 clusters x NB members
-    tab.clear();
-    __syncthreads();
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = c < n;
-    constexpr int P = NB * (NB - 1) / 2;
-    int mem[NB], ty[NB];
-    double xm[NB][3];
-#pragma unroll
-    for (int a = 0; a < NB; a++) {
-        mem[a] = valid ? list[c * NB + a] : 0;
-        ty[a] = A.ctype[mem[a]];
-        for (int k = 0; k < 3; k++) xm[a][k] = A.x[3L * mem[a] + k];
-    }
-    double dist[P], dr[P][3];
-    {
-        int q = 0;
-#pragma unroll
-        for (int a = 0; a < NB; a++)
-#pragma unroll
-            for (int b = a + 1; b < NB; b++, q++) dist[q] = lmp_dist(xm[a], xm[b], dr[q]);
-    }
-    double Ec = 0.0, fo[NB][3], So[6];
-    int flags = 0;
-    bool evaluated = false, tab_err = false;
-    if constexpr (TAB) {
-        if (valid) tab3_cluster(M, T, ty, dist, dr, Ec, fo, So, evaluated, tab_err);
-    } else {
-        if (valid) explicit_cluster<NB, D>(M, ty, dist, dr, Ec, fo, So, flags, evaluated, nullptr);
-    }
-    if (tab_err) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_TAB3);
+    const int nc = *count;
     bool bad = false;
-    double v[6];
-    lmp_order(So, v);
-    // forces of every member, the owner's included, through the LDS table
+    for (int c0 = blockIdx.x * 128; c0 < nc; c0 += gridDim.x * 128) {
+        tab.clear();
+        __syncthreads();
+        const bool valid = c0 + (int)threadIdx.x < nc;
+        const long c = valid ? near[c0 + threadIdx.x] : 0;
+        constexpr int P = NB * (NB - 1) / 2;
+        int mem[NB], ty[NB];
+        double xm[NB][3];
 #pragma unroll
-    for (int a = 0; a < NB; a++) tab.add(evaluated ? mem[a] : -1, fo[a], bad);
-    // per-atom tallies (ev_tally_mb's equal shares): members 1.. by exact
-    // atomics, the owner by runs of equal owners over the wavefront
-    if (A.Eacc || A.Vacc) {
-        if (evaluated)
+        for (int a = 0; a < NB; a++) {
+            mem[a] = valid ? list[c * NB + a] : 0;
+            ty[a] = A.ctype[mem[a]];
+            for (int k = 0; k < 3; k++) xm[a][k] = A.x[3L * mem[a] + k];
+        }
+        double dist[P], dr[P][3];
+        {
+            int q = 0;
 #pragma unroll
-            for (int a = 1; a < NB; a++) {
-                if (A.Eacc) fx_atomic(A.Eacc + 2L * mem[a], Ec / NB, bad);
+            for (int a = 0; a < NB; a++)
+#pragma unroll
+                for (int b = a + 1; b < NB; b++, q++) dist[q] = lmp_dist(xm[a], xm[b], dr[q]);
+        }
+        double Ec = 0.0, fo[NB][3], So[6];
+        int flags = 0;
+        bool evaluated = false, tab_err = false;
+        if constexpr (TAB) {
+            if (valid) tab3_cluster(M, T, ty, dist, dr, Ec, fo, So, evaluated, tab_err);
+        } else {
+            if (valid) explicit_cluster<NB, D>(M, ty, dist, dr, Ec, fo, So, flags, evaluated, nullptr);
+        }
+        if (tab_err) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_TAB3);
+        double v[6];
+        lmp_order(So, v);
+        // forces of every member, the owner's included, through the LDS table
+#pragma unroll
+        for (int a = 0; a < NB; a++) tab.add(evaluated ? mem[a] : -1, fo[a], bad);
+        // per-atom tallies (ev_tally_mb's equal shares): members 1.. by exact
+        // atomics, the owner by runs of equal owners over the wavefront
+        if (A.Eacc || A.Vacc) {
+            if (evaluated)
+#pragma unroll
+                for (int a = 1; a < NB; a++) {
+                    if (A.Eacc) fx_atomic(A.Eacc + 2L * mem[a], Ec / NB, bad);
+                    if (A.Vacc)
+                        for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * mem[a] + k), v[k] / NB, bad);
+                }
+            const int key = evaluated ? mem[0] : -1;
+            if (__ballot(key >= 0)) {
+                const int seg = fx_run_first<64>(key);
+                const int l = threadIdx.x & 63;
+                const int knext = __shfl_down(key, 1, 64);
+                const bool last = key >= 0 && (l == 63 || knext != key);
+                const long o = key >= 0 ? key : 0;
+                if (A.Eacc) lmp_run_add(key, seg, last, Ec / NB, A.Eacc + 2L * o, bad);
                 if (A.Vacc)
-                    for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * mem[a] + k), v[k] / NB, bad);
+                    for (int k = 0; k < 6; k++) lmp_run_add(key, seg, last, v[k] / NB, A.Vacc + 2L * (6L * o + k), bad);
             }
-        const int key = evaluated ? mem[0] : -1;
-        if (__ballot(key >= 0)) {
-            const int seg = fx_run_first<64>(key);
-            const int l = threadIdx.x & 63;
-            const int knext = __shfl_down(key, 1, 64);
-            const bool last = key >= 0 && (l == 63 || knext != key);
-            const long o = key >= 0 ? key : 0;
-            if (A.Eacc) lmp_run_add(key, seg, last, Ec / NB, A.Eacc + 2L * o, bad);
-            if (A.Vacc)
-                for (int k = 0; k < 6; k++) lmp_run_add(key, seg, last, v[k] / NB, A.Vacc + 2L * (6L * o + k), bad);
         }
-    }
-    // global energy and virial: only their sum over all atoms' words is
-    // read, so the wavefront's totals (fourteen integer parts summed at
-    // once) are added to the words of its first evaluated cluster's owner
-    if (A.Gacc) {
-        const unsigned long long on = __ballot(evaluated);
-        if (on) {
-            const int k0 = __builtin_amdgcn_readlane(mem[0], __ffsll((long long)on) - 1);
-            long long x[16];
+        // global energy and virial: only their sum over all atoms' words is
+        // read, so the wavefront's totals (fourteen integer parts summed at
+        // once) are added to the words of its first evaluated cluster's owner
+        if (A.Gacc) {
+            const unsigned long long on = __ballot(evaluated);
+            if (on) {
+                const int k0 = __builtin_amdgcn_readlane(mem[0], __ffsll((long long)on) - 1);
+                long long x[16];
 #pragma unroll
-            for (int k = 0; k < 16; k++) x[k] = 0;
-            if (evaluated) {
-                if (A.eflag_global) fx_split(Ec, x[0], x[1], bad);
-                if (A.vflag_global)
+                for (int k = 0; k < 16; k++) x[k] = 0;
+                if (evaluated) {
+                    if (A.eflag_global) fx_split(Ec, x[0], x[1], bad);
+                    if (A.vflag_global)
 #pragma unroll
-                    for (int k = 0; k < 6; k++) fx_split(v[k], x[2 + 2 * k], x[3 + 2 * k], bad);
+                        for (int k = 0; k < 6; k++) fx_split(v[k], x[2 + 2 * k], x[3 + 2 * k], bad);
+                }
+                const long long t = fx_wave_sums16(x);
+                const int l = threadIdx.x & 63;
+                if (l < 14 && t) atomicAdd(A.Gacc + 14L * k0 + l, (unsigned long long)t);
             }
-            const long long t = fx_wave_sums16(x);
-            const int l = threadIdx.x & 63;
-            if (l < 14 && t) atomicAdd(A.Gacc + 14L * k0 + l, (unsigned long long)t);
         }
+        __syncthreads();
+        tab.flush(A.Facc);
+        __syncthreads();
     }
-    __syncthreads();
-    tab.flush(A.Facc);
     if (bad) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_RANGE);
 }
 
@@ -571,26 +657,32 @@ void launch_lmp_lists(int mode, const chx_lmp_args &A, double pad3, double pad4,
                            cnt4, off3, off4, trips, quads);
 }
 
-void launch_lmp_clusters(int nb, int D, long n, const int *list, const chx_lmp_args &A, const chx_model_dev &M,
-                         const chx_tabs_dev *T, hipStream_t st)
+void launch_lmp_clusters(int nb, int D, long n, const int *list, double rc, int *near, int *count,
+                         const chx_lmp_args &A, const chx_model_dev &M, const chx_tabs_dev *T, hipStream_t st)
 {
     if (n <= 0) return;
-    const dim3 grid((unsigned)((n + 127) / 128)), block(128);
+    const double lim2 = rc * rc * (1.0 + 0x1p-40);
+    const dim3 ngrid((unsigned)((n + NEAR_SPAN - 1) / NEAR_SPAN));
+    if (nb == 3) hipLaunchKernelGGL(k_lmp_near<3>, ngrid, dim3(256), 0, st, n, list, A.x, lim2, near, count);
+    else hipLaunchKernelGGL(k_lmp_near<4>, ngrid, dim3(256), 0, st, n, list, A.x, lim2, near, count);
+    // two workgroups for each of the 1024 the device holds at once (two
+    // wavefronts on each of a CU's SIMDs), fewer for short lists
+    const dim3 grid((unsigned)std::min<long>((n + 127) / 128, 2048)), block(128);
     if (nb == 3 && T && T->ntab3) {
-        hipLaunchKernelGGL((k_lmp_clusters<3, 0, true>), grid, block, 0, st, n, list, A, M, *T);
+        hipLaunchKernelGGL((k_lmp_clusters<3, 0, true>), grid, block, 0, st, count, near, list, A, M, *T);
         return;
     }
-#define X(d)                                                                                         \
-    if (D == d) {                                                                                    \
-        hipLaunchKernelGGL((k_lmp_clusters<3, d, false>), grid, block, 0, st, n, list, A, M, chx_tabs_dev{}); \
-        return;                                                                                      \
+#define X(d)                                                                                                  \
+    if (D == d) {                                                                                             \
+        hipLaunchKernelGGL((k_lmp_clusters<3, d, false>), grid, block, 0, st, count, near, list, A, M, chx_tabs_dev{}); \
+        return;                                                                                               \
     }
     if (nb == 3) { CHX_D3_CASES(X) }
 #undef X
-#define X(d)                                                                                         \
-    if (D == d) {                                                                                    \
-        hipLaunchKernelGGL((k_lmp_clusters<4, d, false>), grid, block, 0, st, n, list, A, M, chx_tabs_dev{}); \
-        return;                                                                                      \
+#define X(d)                                                                                                  \
+    if (D == d) {                                                                                             \
+        hipLaunchKernelGGL((k_lmp_clusters<4, d, false>), grid, block, 0, st, count, near, list, A, M, chx_tabs_dev{}); \
+        return;                                                                                               \
     }
     if (nb == 4) { CHX_D4_CASES(X) }
 #undef X
