@@ -124,34 +124,51 @@ __global__ __launch_bounds__(256) void k_lmp_pair(chx_lmp_args A, chx_model_dev 
 }
 
 // ---------------------------------------------------------------------------
-// Many-body lists, one wavefront per owner ilist[ii].  The owner's row is
+// Many-body lists, four wavefronts per owner ilist[ii].  The owner's row is
 // filtered to J = {j : j != i, tag[j] >= tag[i], d_ij below either padded
 // cutoff}, kept in row order in LDS; every k and l of the reference's loops
-// lies in J.  Triplets come from the (j, k) pairs of J x J in row-major order,
-// quadruplets from each such pair within the 4-body cutoff followed by every
-// l of J, so ballot compaction writes them in the reference's loop order.
-// MODE 0 counts per owner, MODE 1 writes at the scanned offsets.
+// lies in J.  For each a of J a bit row holds the b of J that may follow it
+// (another atom, tag[b] >= tag[a], every distance of (i, a, b) below the
+// padded cutoff).  The triplets are then the set bits of the 3-body rows in
+// row-major order, and the l of a pair (a, b) are the common bits of the
+// 4-body rows of a and b: tag[l] >= tag[b] >= tag[a], both distances and both
+// atoms checked once per pair instead of once per quadruplet, and counting is
+// a population count.  Positions come from the rows' counts, so the lists are
+// written in the reference's loop order.
+//
+// MODE 0 counts per owner, MODE 1 writes at the scanned offsets.  CAP bounds
+// |J|: the small form (29 KB of LDS, five owners a CU) takes owners with at
+// most CAP, the large one those above `lo`; it is launched only when a row is
+// long enough.  1728 atoms at 3.2 g/cc, pads 5.5 / 4.625 A: 67 us
+// to count and 147 us to write, where one wavefront per owner testing every l
+// of every pair took 1286 and 1465 us; the writes are now 53 MB in runs of a
+// few entries per lane.
 // ---------------------------------------------------------------------------
-template <int MODE>
-__global__ __launch_bounds__(64) void k_lmp_lists(chx_lmp_args A, double pad3, double pad4, int has4, int *cnt3,
-                                                  int *cnt4, const long long *off3, const long long *off4,
-                                                  int *trips, int *quads)
+template <int CAP, int MODE>
+__global__ __launch_bounds__(256) void k_lmp_lists(chx_lmp_args A, int lo, double pad3, double pad4, int has4,
+                                                   int *cnt3, int *cnt4, const long long *off3,
+                                                   const long long *off4, int *trips, int *quads)
 {
-    __shared__ int cj[CHX_LMP_CAND], ctag[CHX_LMP_CAND];
-    __shared__ double cx[CHX_LMP_CAND][3], cd[CHX_LMP_CAND];
-    const int ii = blockIdx.x, lane = threadIdx.x;
+    constexpr int W = CAP / 64, LD = W + 1;  // odd row stride: lanes' rows lie in different banks
+    __shared__ double cx[CAP][3], cd[CAP];
+    __shared__ int cj[CAP], ctag[CAP];
+    __shared__ unsigned long long r3[CAP][LD], r4[CAP][LD];
+    __shared__ int row3[CAP], row4[CAP], wsum[4];
+    const int ii = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
     const int i = A.ilist[ii], itag = A.tag[i];
     const double xi[3] = {A.x[3L * i], A.x[3L * i + 1], A.x[3L * i + 2]};
     const int beg = A.nbr_off[ii], n = A.nbr_off[ii + 1] - beg;
     int m = 0;
-    for (int b0 = 0; b0 < n; b0 += 64) {
+    for (int b0 = 0; b0 < n; b0 += 256) {
         bool v = false;
-        int j = 0;
+        int j = 0, tj = 0;
         double xj[3] = {0, 0, 0}, d = 0.0;
-        if (b0 + lane < n) {
-            j = A.nbr[beg + b0 + lane];
-            if (j != i && A.tag[j] >= itag) {
+        if (b0 + tid < n) {
+            j = A.nbr[beg + b0 + tid];
+            tj = A.tag[j];
+            if (j != i && tj >= itag) {
                 xj[0] = A.x[3L * j]; xj[1] = A.x[3L * j + 1]; xj[2] = A.x[3L * j + 2];
                 double dr[3];
                 d = lmp_dist(xi, xj, dr);
@@ -159,75 +176,135 @@ __global__ __launch_bounds__(64) void k_lmp_lists(chx_lmp_args A, double pad3, d
             }
         }
         const unsigned long long bal = __ballot(v);
-        const int r = m + __popcll(bal & below);
-        if (v && r < CHX_LMP_CAND) {
+        if (lane == 0) wsum[wv] = __popcll(bal);
+        __syncthreads();
+        int r = m + __popcll(bal & below);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            r += w < wv ? wsum[w] : 0;
+            m += wsum[w];
+        }
+        if (v && r < CAP) {
             cj[r] = j;
-            ctag[r] = A.tag[j];
+            ctag[r] = tj;
             cx[r][0] = xj[0]; cx[r][1] = xj[1]; cx[r][2] = xj[2];
             cd[r] = d;
         }
-        m += __popcll(bal);
+        __syncthreads();
     }
-    if (m > CHX_LMP_CAND) {
-        if (lane == 0) {
+    if (m <= lo) return;
+    if (m > CAP) {
+        if (CAP == CHX_LMP_CAND && tid == 0) {
             atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_CAND);
             atomicMax(&A.status[CHX_LMP_ST_MAXCAND], m);
         }
         return;
     }
-    __syncthreads();
-    long long c3 = 0, c4 = 0;
-    const long long o3 = MODE ? off3[ii] : 0, o4 = MODE ? off4[ii] : 0;
-    const int total = m * m;
-    for (int p0 = 0; p0 < total; p0 += 64) {
-        const int p = p0 + lane;
-        bool v3 = false, v4 = false;
-        int a = 0, b = 0;
-        if (p < total) {
-            a = p / m;
-            b = p - a * m;
-            if (cj[a] != cj[b] && ctag[b] >= ctag[a]) {
+    const int mw = (m + 63) >> 6;
+    for (int a = wv; a < m; a += 4) {
+        const double da = cd[a];
+        for (int w = 0; w < mw; w++) {
+            const int b = w * 64 + lane;
+            bool v3 = false, v4 = false;
+            if (b < m && cj[a] != cj[b] && ctag[b] >= ctag[a]) {
                 double dr[3];
                 const double dab = lmp_dist(cx[a], cx[b], dr);
-                const double da = cd[a], db = cd[b];
+                const double db = cd[b];
                 v3 = da < pad3 && db < pad3 && dab < pad3;
                 v4 = has4 && da < pad4 && db < pad4 && dab < pad4;
             }
-        }
-        const unsigned long long b3 = __ballot(v3);
-        if (MODE && v3) {
-            int *t = trips + 3 * (o3 + c3 + __popcll(b3 & below));
-            t[0] = i; t[1] = cj[a]; t[2] = cj[b];
-        }
-        c3 += __popcll(b3);
-        unsigned long long b4 = __ballot(v4);
-        while (b4) {
-            const int t = __ffsll((long long)b4) - 1;
-            b4 &= b4 - 1;
-            const int pt = p0 + t, at = pt / m, bt = pt - at * m;
-            const int ja = cj[at], jb = cj[bt], tb = ctag[bt];
-            for (int q0 = 0; q0 < m; q0 += 64) {
-                const int q = q0 + lane;
-                bool v = false;
-                if (q < m) {
-                    const int l = cj[q];
-                    if (l != ja && l != jb && ctag[q] >= tb && cd[q] < pad4) {
-                        double dr[3];
-                        v = lmp_dist(cx[at], cx[q], dr) < pad4 && lmp_dist(cx[bt], cx[q], dr) < pad4;
-                    }
-                }
-                const unsigned long long bl = __ballot(v);
-                if (MODE && v) {
-                    int *u = quads + 4 * (o4 + c4 + __popcll(bl & below));
-                    u[0] = i; u[1] = ja; u[2] = jb; u[3] = cj[q];
-                }
-                c4 += __popcll(bl);
+            const unsigned long long b3 = __ballot(v3), b4 = __ballot(v4);
+            if (lane == 0) {
+                r3[a][w] = b3;
+                r4[a][w] = b4;
             }
         }
     }
-    if (!MODE && lane == 0) {
-        cnt3[ii] = (int)c3;
-        cnt4[ii] = (int)c4;
+    __syncthreads();
+    // quadruplets of the pair (a, b): the common followers of a and b
+    auto common = [&](int a, int b) {
+        int c = 0;
+        for (int w = 0; w < mw; w++) c += __popcll(r4[a][w] & r4[b][w]);
+        return c;
+    };
+    // clusters of each row
+    for (int a = wv; a < m; a += 4) {
+        int c3 = 0, c4 = 0;
+        for (int w = 0; w < mw; w++) {
+            c3 += __popcll(r3[a][w]);
+            const unsigned long long b4 = r4[a][w];
+            if (b4 == 0) continue;
+            if ((b4 >> lane) & 1) c4 += common(a, w * 64 + lane);
+        }
+        for (int s = 1; s < 64; s <<= 1) c4 += __shfl_xor(c4, s, 64);
+        if (lane == 0) {
+            row3[a] = c3;
+            row4[a] = c4;
+        }
+    }
+    __syncthreads();
+    // rows' offsets (exclusive) and totals, by the first wavefront
+    if (wv == 0) {
+        int t3 = 0, t4 = 0;
+        for (int w = 0; w < mw; w++) {
+            const int a = w * 64 + lane;
+            const int c3 = a < m ? row3[a] : 0, c4 = a < m ? row4[a] : 0;
+            int s3 = c3, s4 = c4;
+            for (int s = 1; s < 64; s <<= 1) {
+                const int u3 = __shfl_up(s3, s, 64), u4 = __shfl_up(s4, s, 64);
+                if (lane >= s) {
+                    s3 += u3;
+                    s4 += u4;
+                }
+            }
+            if (a < m) {
+                row3[a] = t3 + s3 - c3;
+                row4[a] = t4 + s4 - c4;
+            }
+            t3 += __shfl(s3, 63, 64);
+            t4 += __shfl(s4, 63, 64);
+        }
+        if (MODE == 0 && lane == 0) {
+            cnt3[ii] = t3;
+            cnt4[ii] = t4;
+        }
+    }
+    if (MODE == 0) return;
+    __syncthreads();
+    const long long o3 = off3[ii], o4 = off4[ii];
+    for (int a = wv; a < m; a += 4) {
+        const int ja = cj[a];
+        int p3 = row3[a], p4 = row4[a];
+        for (int w = 0; w < mw; w++) {
+            const int b = w * 64 + lane;
+            const unsigned long long b3 = r3[a][w], b4 = r4[a][w];
+            if ((b3 >> lane) & 1) {
+                int *t = trips + 3 * (o3 + p3 + __popcll(b3 & below));
+                t[0] = i; t[1] = ja; t[2] = cj[b];
+            }
+            p3 += __popcll(b3);
+            if (b4 == 0) continue;
+            const bool on = (b4 >> lane) & 1;
+            const int c = on ? common(a, b) : 0;
+            int s4 = c;
+            for (int s = 1; s < 64; s <<= 1) {
+                const int u4 = __shfl_up(s4, s, 64);
+                if (lane >= s) s4 += u4;
+            }
+            // each lane writes its pair's quadruplets, one consecutive run
+            if (c) {
+                int4 *u = reinterpret_cast<int4 *>(quads) + (o4 + p4 + s4 - c);
+                const int jb = cj[b];
+                for (int y = 0; y < mw; y++) {
+                    unsigned long long l = r4[a][y] & r4[b][y];
+                    while (l) {
+                        *u++ = make_int4(i, ja, jb, cj[y * 64 + __ffsll((long long)l) - 1]);
+                        l &= l - 1;
+                    }
+                }
+            }
+            p4 += __shfl(s4, 63, 64);
+        }
     }
 }
 
@@ -645,16 +722,23 @@ void launch_lmp_pair(const chx_lmp_args &A, const chx_model_dev &M, const chx_ta
     else hipLaunchKernelGGL(k_lmp_pair<false>, grid, block, 0, st, A, M, chx_tabs_dev{});
 }
 
-void launch_lmp_lists(int mode, const chx_lmp_args &A, double pad3, double pad4, int has4, int *cnt3, int *cnt4,
-                      const long long *off3, const long long *off4, int *trips, int *quads, hipStream_t st)
+void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, double pad3, double pad4, int has4, int *cnt3,
+                      int *cnt4, const long long *off3, const long long *off4, int *trips, int *quads, hipStream_t st)
 {
     if (A.inum <= 0) return;
-    if (mode == 0)
-        hipLaunchKernelGGL(k_lmp_lists<0>, dim3((unsigned)A.inum), dim3(64), 0, st, A, pad3, pad4, has4, cnt3,
-                           cnt4, off3, off4, trips, quads);
-    else
-        hipLaunchKernelGGL(k_lmp_lists<1>, dim3((unsigned)A.inum), dim3(64), 0, st, A, pad3, pad4, has4, cnt3,
-                           cnt4, off3, off4, trips, quads);
+    constexpr int SMALL = CHX_LMP_CAND / 2;
+    const dim3 grid((unsigned)A.inum), block(256);
+#define L(CAP_, MODE_, LO_)                                                                                    \
+    hipLaunchKernelGGL((k_lmp_lists<CAP_, MODE_>), grid, block, 0, st, A, LO_, pad3, pad4, has4, cnt3, cnt4, off3, \
+                       off4, trips, quads)
+    if (mode == 0) {
+        L(SMALL, 0, -1);
+        if (max_row > SMALL) L(CHX_LMP_CAND, 0, SMALL);
+    } else {
+        L(SMALL, 1, -1);
+        if (max_row > SMALL) L(CHX_LMP_CAND, 1, SMALL);
+    }
+#undef L
 }
 
 void launch_lmp_clusters(int nb, int D, long n, const int *list, double rc, int *near, int *count,

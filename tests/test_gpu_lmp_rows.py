@@ -1,0 +1,39 @@
+"""The pair style's list kernel where its bit rows end: owners whose filtered
+rows hold just below, at and above 64 and 256 candidates (word and working-set
+edges, the large form included), list entries compared exactly with the
+oracle's."""
+import numpy as np
+import pytest
+
+from chimes_calculator_amd import workloads as W
+from lmp_setup import LmpSystem
+from oracle_bindings import LmpOracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("natoms,rc4", [(2, 3.5), (64, 3.5), (65, 3.5), (66, 0.9), (129, 2.0), (257, 1.2), (259, 1.2)])
+def test_rows(tmp_path, natoms, rc4):
+    from chimes_calculator_amd import GpuModel, LmpPair
+    # natoms atoms in a ball of 2.2 A: the owner of the lowest tag has all others in its row
+    m = W.Model("ball", ["C"], (4, 3, 3), (5.0, 4.0, rc4), {frozenset(("C",)): 0.05}, seed=natoms)
+    pf = m.write(str(tmp_path / "ball.txt"))
+    rng = np.random.default_rng(natoms)
+    v = rng.normal(size=(natoms, 3))
+    x = 10.0 + v / np.linalg.norm(v, axis=1)[:, None] * 2.2 * rng.random((natoms, 1)) ** (1.0 / 3.0)
+    O = LmpOracle(pf)
+    S = LmpSystem(x, np.ones(natoms, np.int32), rng.permutation(natoms).astype(np.int32) + 1, np.zeros(3),
+                  np.full(3, 20.0), [0], O.rc2(), 0.0, shuffle_seed=1)
+    keep = 3 if natoms > 100 else natoms  # owners: the lists of a few low tags are long enough
+    S.ilist = np.argsort(S.tag[: S.nlocal])[:keep].astype(np.int32)
+    rows = [S.nbr[S.nbr_off[i]:S.nbr_off[i + 1]] for i in S.ilist]
+    S.inum, S.nbr = keep, np.concatenate(rows).astype(np.int32)
+    S.nbr_off = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    trips, quads = O.build_lists(S)
+    model = GpuModel(pf)
+    P = LmpPair(model, {1: W.MASS["C"]})
+    P.build_mb_neighlists(S.x, S.tag, S.ilist, S.numneigh, S.nbr_off, S.nbr, skin=0.0)
+    g3, g4 = P.mb_lists()
+    assert np.array_equal(g3, trips) and np.array_equal(g4, quads), (len(trips), len(quads))
+    P.close()
+    model.close()
