@@ -11,6 +11,9 @@ namespace chx {
 // Longest filtered neighbour row (images within the padded many-body
 // cutoffs, tag not below the owner's) the list kernel holds in LDS.
 constexpr int CHX_LMP_CAND = 512;
+// copies of the global energy and virial sums, one 128-byte line each, picked
+// by workgroup
+constexpr int CHX_LMP_GSLOTS = 256;
 // status words of the adapter
 enum : int {
     CHX_LMP_ST_FLAGS = 0,
@@ -32,7 +35,7 @@ struct chx_lmp_args {
     unsigned long long *Facc;  // [nall * 3 * 2] fixed-point forces
     unsigned long long *Eacc;  // [nall * 2] per-atom energy, or null
     unsigned long long *Vacc;  // [nall * 6 * 2] per-atom virial (LAMMPS order), or null
-    unsigned long long *Gacc;  // [nall * 7 * 2] partial sums of the global energy + virial (only the total over all atoms is read), or null
+    unsigned long long *Gacc;  // [CHX_LMP_GSLOTS][16] copies of the global energy + virial (7 (hi, lo) pairs), or null
     int *status;               // [CHX_LMP_ST_WORDS]
     int eflag_global, vflag_global;
 };
@@ -53,9 +56,7 @@ void launch_lmp_clusters(int nb, int D, long n, const int *list, double rc, int 
 // nb(nb-1)/2 distances then nb types).
 void launch_lmp_fp_rows(int nb, int mode, long n, const int *list, const chx_lmp_args &A, const chx_model_dev &M,
                         int *blk_cnt, const long long *blk_off, double *rows, hipStream_t st);
-// F[nall*3], eatom[nall] (if Eacc), vatom[nall*6] (if Vacc), glob[7] (if
-// Gacc; gsum[14] and *done zeroed scratch of the global reduction)
-void launch_lmp_out(const chx_lmp_args &A, double *F, double *eatom, double *vatom, double *glob,
-                    unsigned long long *gsum, int *done, hipStream_t st);
+// F[nall*3], eatom[nall] (if Eacc), vatom[nall*6] (if Vacc), glob[7] (if Gacc)
+void launch_lmp_out(const chx_lmp_args &A, double *F, double *eatom, double *vatom, double *glob, hipStream_t st);
 
 }  // namespace chx

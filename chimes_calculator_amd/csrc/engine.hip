@@ -2329,13 +2329,12 @@ int chx_lmp_compute(chx_lmp *p, int nall, const double *x, const int *type, cons
         if (rebuild) lmp_build(p, skin);
         HIPCHK(hipEventRecord(p->ev[2], st));
         const chx_model *m = p->m;
-        // accumulators: forces, per-atom energy, per-atom virial, per-owner global
+        // accumulators: forces, per-atom energy, per-atom virial, copies of the global sums
         const size_t nF = (size_t)nall * 6, nE = eflag_atom ? (size_t)nall * 2 : 0,
                      nV = vflag_atom ? (size_t)nall * 12 : 0,
-                     nG = (eflag_global || vflag_global) ? (size_t)nall * 14 : 0;
-        // plus the global reduction's sums (14 words) and block counter (1)
-        p->acc.ensure(nF + nE + nV + nG + 15);
-        HIPCHK(hipMemsetAsync(p->acc.p, 0, sizeof(unsigned long long) * (nF + nE + nV + nG + 15), st));
+                     nG = (eflag_global || vflag_global) ? (size_t)CHX_LMP_GSLOTS * 16 : 0;
+        p->acc.ensure(nF + nE + nV + nG);
+        HIPCHK(hipMemsetAsync(p->acc.p, 0, sizeof(unsigned long long) * (nF + nE + nV + nG), st));
         chx_lmp_args A = p->args();
         A.Facc = p->acc.p;
         A.Eacc = nE ? A.Facc + nF : nullptr;
@@ -2359,8 +2358,7 @@ int chx_lmp_compute(chx_lmp *p, int nall, const double *x, const int *type, cons
         p->out.ensure(nout + CHX_LMP_ST_WORDS);
         double *F = p->out.p, *Ea = F + (size_t)nall * 3, *Va = Ea + (nE ? nall : 0),
                *G = Va + (nV ? (size_t)nall * 6 : 0);
-        unsigned long long *gsum = p->acc.p + nF + nE + nV + nG;
-        launch_lmp_out(A, F, nE ? Ea : nullptr, nV ? Va : nullptr, G, gsum, (int *)(gsum + 14), st);
+        launch_lmp_out(A, F, nE ? Ea : nullptr, nV ? Va : nullptr, G, st);
         HIPCHK(hipGetLastError());
         HIPCHK(hipMemcpyAsync(p->out.p + nout, p->status.p, sizeof(int) * CHX_LMP_ST_WORDS, hipMemcpyDeviceToDevice,
                               st));

@@ -3,8 +3,7 @@
 //   k_lmp_pair      1- and 2-body loops of PairCHIMES::compute (567-656)
 //   k_lmp_lists     PairCHIMES::build_mb_neighlists (321-478)
 //   k_lmp_clusters  3- and 4-body loops (673-829) over those lists
-//   k_lmp_out       fixed-point accumulators -> forces and per-atom tallies
-//   k_lmp_global    global energy and virial
+//   k_lmp_out       fixed-point accumulators -> forces and tallies
 // Every tally of Pair::ev_tally_mb (etc/lmp/etc/pair.cpp:1425-1482) is added
 // in the exact fixed-point form of the batch pipeline, so results do not
 // depend on the order of the lists or on the kernel schedule.
@@ -35,90 +34,215 @@ __device__ __forceinline__ void lmp_order(const double (&s)[6], double (&v)[6])
     v[3] = s[1]; v[4] = s[2]; v[5] = s[4];
 }
 
+// Per-workgroup LDS table of the atoms a tile adds to, the pair style's form
+// of fx_table: three force components per atom and, when the step asks for
+// per-atom tallies, its energy and six virial terms, as (hi, lo) words in
+// dynamic LDS.  An atom that finds no slot within LMP_PROBES goes straight to
+// memory.
+constexpr int LMP_PROBES = 32;
+
+struct lmp_table {
+    int cap, nw;               // slots (a power of two), words per slot: 6 or 20
+    int *key;
+    unsigned long long *val;   // [cap][nw]: 3 forces, energy, 6 virial terms
+    __host__ __device__ static size_t bytes(int cap, int nw) { return (size_t)cap * (8 * nw + 4); }
+    __device__ __forceinline__ lmp_table(char *lds, int cap_, bool tally) : cap(cap_), nw(tally ? 20 : 6)
+    {
+        val = reinterpret_cast<unsigned long long *>(lds);
+        key = reinterpret_cast<int *>(val + (size_t)cap * nw);
+    }
+    // all threads; a barrier must follow before use
+    __device__ __forceinline__ void clear()
+    {
+        for (int s = threadIdx.x; s < cap; s += blockDim.x) key[s] = -1;
+        for (int s = threadIdx.x; s < cap * nw; s += blockDim.x) val[s] = 0ull;
+    }
+    // force F and (tallying) energy share e and virial share w * v of an atom
+    __device__ __forceinline__ void add(int atom, const double (&F)[3], double e, const double (&v)[6],
+                                        const chx_lmp_args &A, bool &bad)
+    {
+        if (atom < 0) return;
+        int s = (int)((((unsigned)atom * 2654435761u) >> 8) & (cap - 1));
+        bool found = false;
+        for (int probe = 0; probe < LMP_PROBES; probe++) {
+            const int prev = atomicCAS(&key[s], -1, atom);
+            if (prev == -1 || prev == atom) { found = true; break; }
+            s = (s + 1) & (cap - 1);
+        }
+        if (!found) {
+            for (int k = 0; k < 3; k++) fx_atomic(A.Facc + 2L * (3L * atom + k), F[k], bad);
+            if (A.Eacc) fx_atomic(A.Eacc + 2L * atom, e, bad);
+            if (A.Vacc)
+                for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * atom + k), v[k], bad);
+            return;
+        }
+        unsigned long long *a = val + s * nw;
+#pragma unroll
+        for (int k = 0; k < 3; k++) fx_atomic(a + 2 * k, F[k], bad);
+        if (A.Eacc) fx_atomic(a + 6, e, bad);
+        if (A.Vacc)
+#pragma unroll
+            for (int k = 0; k < 6; k++) fx_atomic(a + 8 + 2 * k, v[k], bad);
+    }
+    // all threads, after a barrier
+    __device__ __forceinline__ void flush(const chx_lmp_args &A)
+    {
+        for (int t = threadIdx.x; t < cap * nw; t += blockDim.x) {
+            const int s = t / nw, k = t - s * nw;
+            const unsigned long long w = val[t];
+            if (key[s] < 0 || !w) continue;
+            const long atom = key[s];
+            unsigned long long *g = k < 6 ? A.Facc + 6 * atom + k
+                                          : (k < 8 ? A.Eacc + 2 * atom + (k - 6) : A.Vacc + 12 * atom + (k - 8));
+            atomicAdd(g, w);
+        }
+    }
+};
+
+// Adds the wavefront's energies and virials (lanes of on) into copy `slot` of
+// the global sums: fourteen integer parts summed over the lanes at once.
+__device__ __forceinline__ void lmp_global_add(const chx_lmp_args &A, bool on, double E, const double (&v)[6],
+                                               int slot, bool &bad)
+{
+    if (!A.Gacc || __ballot(on) == 0) return;
+    long long x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = 0;
+    if (on) {
+        if (A.eflag_global) fx_split(E, x[0], x[1], bad);
+        if (A.vflag_global)
+#pragma unroll
+            for (int k = 0; k < 6; k++) fx_split(v[k], x[2 + 2 * k], x[3 + 2 * k], bad);
+    }
+    const long long t = fx_wave_sums16(x);
+    const int l = threadIdx.x & 63;
+    if (l < 14 && t) atomicAdd(A.Gacc + (long)slot * 16 + l, (unsigned long long)t);
+}
+
+// Sum of a double over the wavefront, in one fixed order.
+__device__ __forceinline__ double lmp_wave_sum(double x)
+{
+    const long long r = __double_as_longlong(group_sum<16>(x));  // each row's total on its last lane
+    const double s0 = __longlong_as_double(readlane_i64(r, 15)), s1 = __longlong_as_double(readlane_i64(r, 31)),
+                 s2 = __longlong_as_double(readlane_i64(r, 47)), s3 = __longlong_as_double(readlane_i64(r, 63));
+    return (s0 + s1) + (s2 + s3);
+}
+
 // ---------------------------------------------------------------------------
-// 1- and 2-body: sixteen lanes per owner ilist[ii]; lane l takes row entries
-// l, l + 16, ...  Pairs with tag[j] > tag[i] only (pair_chimes.cpp:603).  The
-// owner's force and tallies are summed over its lanes in double in that fixed
-// order and added exactly once; the partner's are added per pair.  TAB: the
-// pair's energy and force scalar come from its table (compute_2B_tab,
-// chimesFF.cpp:1782-1856: cutoff test, table lookups, no penalty term).
+// 1- and 2-body: one wavefront per owner ilist[ii], four owners per
+// workgroup.  Pairs with tag[j] > tag[i] only (pair_chimes.cpp:603).  A row
+// reaches one skin past the cutoff and half of it has lower tags, so three
+// quarters of its entries are skipped: the wavefront queues the entries that
+// count, in row order, and evaluates 64 at a time, where lanes striding over
+// the row each did a few of many passes.  The owner's force and tallies are
+// summed over its lanes in double in that fixed order and added exactly once;
+// the partners' go through the workgroup's table.  4096 carbon atoms, order
+// 20, 184-entry rows: 40 us with energy and virial, where sixteen striding
+// lanes per owner and atomics to memory took 73 us (1728 atoms with per-atom
+// tallies: 30 us, before 102 us).  TAB: the pair's energy and force scalar
+// come from its table (compute_2B_tab, chimesFF.cpp:1782-1856: cutoff test,
+// table lookups, no penalty term).
 // ---------------------------------------------------------------------------
+constexpr int LMP_PAIR_SLOTS = 256;
+
 template <bool TAB>
 __global__ __launch_bounds__(256) void k_lmp_pair(chx_lmp_args A, chx_model_dev M, chx_tabs_dev T)
 {
-    const int sub = threadIdx.x & 15;
-    const int ii = (int)(blockIdx.x * 16 + (threadIdx.x >> 4));
-    if (ii >= A.inum) return;  // whole groups of sixteen leave together
-    const int i = A.ilist[ii];
-    const int itag = A.tag[i], ti = A.ctype[i];
-    const double xi[3] = {A.x[3L * i], A.x[3L * i + 1], A.x[3L * i + 2]};
-    // owner force, owner energy share, owner virial share, global energy, global virial
-    double fi[3] = {0, 0, 0}, ea = 0.0, va[6] = {0, 0, 0, 0, 0, 0}, ge = 0.0, gv[6] = {0, 0, 0, 0, 0, 0};
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    __shared__ int queue[4][128];
+    const bool tally = A.Eacc || A.Vacc;
+    lmp_table tab(lds, LMP_PAIR_SLOTS, tally);
+    tab.clear();
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const int ii = (int)(blockIdx.x * 4 + wv);
     bool bad = false, tab_err = false;
-    int flags = 0;
-    const int beg = A.nbr_off[ii], end = A.nbr_off[ii + 1];
-    for (int q = beg + sub; q < end; q += 16) {
-        const int j = A.nbr[q];
-        if (A.tag[j] <= itag) continue;
-        const double xj[3] = {A.x[3L * j], A.x[3L * j + 1], A.x[3L * j + 2]};
-        double dr[3];
-        const double r = lmp_dist(xi, xj, dr);
-        const int pt = M.pairmap[ti * M.nt + A.ctype[j]];
-        double E, fs;
-        if constexpr (TAB) {
-            if (r >= M.slots2[pt].rout) continue;
-            tab2_lookup(T, pt, r, E, fs, tab_err);
-        } else {
-            eval_pair(r, M.slots2[pt], M.c2 + (long)pt * (M.order[0] + 1), M.order[0], M.tersoff, M.fcut_var,
-                      M.pen_dist, M.pen_scale, E, fs, flags);
-            if (r >= M.slots2[pt].rout) continue;
-        }
-        const double F[3] = {fs * dr[0], fs * dr[1], fs * dr[2]};
-        const double s[6] = {-(fs * (dr[0] * dr[0])), -(fs * (dr[0] * dr[1])), -(fs * (dr[0] * dr[2])),
-                             -(fs * (dr[1] * dr[1])), -(fs * (dr[1] * dr[2])), -(fs * (dr[2] * dr[2]))};
-        double v[6];
-        lmp_order(s, v);
-        for (int k = 0; k < 3; k++) {
-            fi[k] += F[k];
-            fx_atomic(A.Facc + 2L * (3L * j + k), -F[k], bad);
-        }
-        ge += E;
-        ea += E / 2;
-        if (A.Eacc) fx_atomic(A.Eacc + 2L * j, E / 2, bad);
-        for (int k = 0; k < 6; k++) {
-            gv[k] += v[k];
-            va[k] += v[k] / 2;
-            if (A.Vacc) fx_atomic(A.Vacc + 2L * (6L * j + k), v[k] / 2, bad);
-        }
-    }
+    if (ii < A.inum) {
+        const int i = A.ilist[ii];
+        const int itag = A.tag[i], ti = A.ctype[i];
+        const double xi[3] = {A.x[3L * i], A.x[3L * i + 1], A.x[3L * i + 2]};
+        // owner force, energy and virial of the pairs (halves go to each atom)
+        double acc[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        int flags = 0, nq = 0;
+        // the first cnt queued partners, one per lane
+        auto batch = [&](int cnt) {
+            double E = 0.0, v[6] = {0, 0, 0, 0, 0, 0};
+            if (lane < cnt) {
+                const int j = queue[wv][lane];
+                const double xj[3] = {A.x[3L * j], A.x[3L * j + 1], A.x[3L * j + 2]};
+                double dr[3], fs;
+                const double r = lmp_dist(xi, xj, dr);
+                const int pt = M.pairmap[ti * M.nt + A.ctype[j]];
+                if constexpr (TAB) tab2_lookup(T, pt, r, E, fs, tab_err);
+                else
+                    eval_pair(r, M.slots2[pt], M.c2 + (long)pt * (M.order[0] + 1), M.order[0], M.tersoff, M.fcut_var,
+                              M.pen_dist, M.pen_scale, E, fs, flags);
+                const double F[3] = {fs * dr[0], fs * dr[1], fs * dr[2]};
+                const double s[6] = {-(fs * (dr[0] * dr[0])), -(fs * (dr[0] * dr[1])), -(fs * (dr[0] * dr[2])),
+                                     -(fs * (dr[1] * dr[1])), -(fs * (dr[1] * dr[2])), -(fs * (dr[2] * dr[2]))};
+                lmp_order(s, v);
+                const double Fj[3] = {-F[0], -F[1], -F[2]};
+                const double vj[6] = {v[0] / 2, v[1] / 2, v[2] / 2, v[3] / 2, v[4] / 2, v[5] / 2};
+                tab.add(j, Fj, E / 2, vj, A, bad);
 #pragma unroll
-    for (int w = 8; w >= 1; w >>= 1) {
-        for (int k = 0; k < 3; k++) fi[k] += __shfl_xor(fi[k], w, 64);
-        ea += __shfl_xor(ea, w, 64);
-        ge += __shfl_xor(ge, w, 64);
-        for (int k = 0; k < 6; k++) {
-            va[k] += __shfl_xor(va[k], w, 64);
-            gv[k] += __shfl_xor(gv[k], w, 64);
-        }
-    }
-    if (sub == 0) {
-        const double e1 = M.eoff[ti];  // compute_1B, tallied for one atom
-        for (int k = 0; k < 3; k++) fx_atomic(A.Facc + 2L * (3L * i + k), fi[k], bad);
-        if (A.Eacc) {
-            fx_atomic(A.Eacc + 2L * i, e1, bad);
-            fx_atomic(A.Eacc + 2L * i, ea, bad);
-        }
-        if (A.Vacc)
-            for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * i + k), va[k], bad);
-        if (A.Gacc) {
-            if (A.eflag_global) {
-                fx_atomic(A.Gacc + 2L * (7L * i), e1, bad);
-                fx_atomic(A.Gacc + 2L * (7L * i), ge, bad);
+                for (int k = 0; k < 3; k++) acc[k] += F[k];
+                acc[3] += E;
+#pragma unroll
+                for (int k = 0; k < 6; k++) acc[4 + k] += v[k];
             }
-            if (A.vflag_global)
-                for (int k = 0; k < 6; k++) fx_atomic(A.Gacc + 2L * (7L * i + 1 + k), gv[k], bad);
+        };
+        const int beg = A.nbr_off[ii], end = A.nbr_off[ii + 1];
+        for (int q0 = beg; q0 < end; q0 += 64) {
+            bool in = false;
+            int j = 0;
+            if (q0 + lane < end) {
+                j = A.nbr[q0 + lane];
+                if (A.tag[j] > itag) {
+                    const double xj[3] = {A.x[3L * j], A.x[3L * j + 1], A.x[3L * j + 2]};
+                    double dr[3];
+                    in = !(lmp_dist(xi, xj, dr) >= M.slots2[M.pairmap[ti * M.nt + A.ctype[j]]].rout);
+                }
+            }
+            const unsigned long long b = __ballot(in);
+            if (in) queue[wv][nq + __popcll(b & below)] = j;
+            nq += __popcll(b);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (nq >= 64) {
+                batch(64);
+                nq -= 64;
+                const int rest = lane < nq ? queue[wv][64 + lane] : 0;
+                __builtin_amdgcn_wave_barrier();
+                if (lane < nq) queue[wv][lane] = rest;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
+        if (nq) batch(nq);
+        double tot[10];
+#pragma unroll
+        for (int k = 0; k < 10; k++) tot[k] = lmp_wave_sum(acc[k]);
+        const double e1 = M.eoff[ti];  // compute_1B, tallied for one atom
+        const double v[6] = {tot[4], tot[5], tot[6], tot[7], tot[8], tot[9]};
+        if (lane == 0) {
+            for (int k = 0; k < 3; k++) fx_atomic(A.Facc + 2L * (3L * i + k), tot[k], bad);
+            if (A.Eacc) {
+                fx_atomic(A.Eacc + 2L * i, e1, bad);
+                fx_atomic(A.Eacc + 2L * i, tot[3] / 2, bad);
+            }
+            if (A.Vacc)
+                for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * i + k), v[k] / 2, bad);
+        }
+        // lane 0 the pairs' energy and virial, lane 1 the 1-body energy
+        const double z[6] = {0, 0, 0, 0, 0, 0}, ev = lane ? e1 : tot[3];
+        double gv[6];
+#pragma unroll
+        for (int k = 0; k < 6; k++) gv[k] = lane ? z[k] : v[k];
+        lmp_global_add(A, lane < 2, ev, gv, blockIdx.x & (CHX_LMP_GSLOTS - 1), bad);
     }
+    __syncthreads();
+    tab.flush(A);
     if (bad) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_RANGE);
     if (tab_err) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_TAB2);
 }
@@ -315,20 +439,6 @@ __global__ __launch_bounds__(256) void k_lmp_lists(chx_lmp_args A, int lo, doubl
 // the tallies of ev_tally_mb (energy and virial shared equally by the
 // members; the global part kept per owner atom).
 // ---------------------------------------------------------------------------
-// One value of the owner atom: summed over the wavefront's runs of equal keys
-// (the lists are sorted by owner) and added by each run's last lane at a.
-__device__ __forceinline__ void lmp_run_add(int key, int seg, bool last, double v, unsigned long long *a, bool &bad)
-{
-    long long x[2] = {0, 0};
-    if (key >= 0) fx_split(v, x[0], x[1], bad);
-    fx_run_scan<64, 2>(x, seg);
-    if (last) {
-        if (x[0]) atomicAdd(a, (unsigned long long)x[0]);
-        if (x[1]) atomicAdd(a + 1, (unsigned long long)x[1]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 // compute_3B_tab (chimesFF.cpp:2183-2313): exclusion and the cutoffs of the
 // mapped slots as compute_3B, then the table at the runtime pair distances
 // (ij, ik, jk; get_tab_3B's sort is not executed, 2459-2470); forces and
@@ -384,6 +494,7 @@ __device__ __forceinline__ void tab3_cluster(const chx_model_dev &M, const chx_t
 // Bound by the gathers of the members' positions (L2).
 // ---------------------------------------------------------------------------
 constexpr int NEAR_SPAN = 2048;
+constexpr int LMP_TILE_SLOTS = 256;
 
 template <int NB>
 __global__ __launch_bounds__(256) void k_lmp_near(long n, const int *__restrict__ list,
@@ -450,13 +561,17 @@ __global__ __launch_bounds__(256) void k_lmp_near(long n, const int *__restrict_
 // them 128 at a time, since the host does not know their number.  4096 carbon
 // atoms at 3.2 g/cc, orders 5 / 3: one entry per lane over the whole lists took
 // 269 us (triplets) and 890 us (quadruplets), and a step of the pair style
-// 1426 us; selection and evaluation together leave a step of 504 us.
+// 1426 us; selection and evaluation together leave a step of 504 us.  With the
+// per-atom tallies through the table too, 1728 atoms take 66 and 57 us (337 and
+// 172 us with those in atomics to memory).
 template <int NB, int D, bool TAB>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k_lmp_clusters(const int *__restrict__ count, const int *__restrict__ near, const int *__restrict__ list, chx_lmp_args A,
                                                       chx_model_dev M, chx_tabs_dev T)
 {
-    // the members' forces of the workgroup's clusters, merged per atom
-    __shared__ fx_table<512> tab;  // >= 128 clusters x NB members
+    // forces and per-atom tallies of the workgroup's clusters, merged per atom
+    // (a tile of consecutive clusters touches one or two hundred atoms)
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    lmp_table tab(lds, LMP_TILE_SLOTS, A.Eacc || A.Vacc);
     const int nc = *count;
     bool bad = false;
     for (int c0 = blockIdx.x * 128; c0 < nc; c0 += gridDim.x * 128) {
@@ -492,65 +607,53 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k
         if (tab_err) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_TAB3);
         double v[6];
         lmp_order(So, v);
-        // forces of every member, the owner's included, through the LDS table
+        // every member's force and share of the tallies (ev_tally_mb), the
+        // owner's included, through the LDS table
+        const double e = Ec / NB, vs[6] = {v[0] / NB, v[1] / NB, v[2] / NB, v[3] / NB, v[4] / NB, v[5] / NB};
 #pragma unroll
-        for (int a = 0; a < NB; a++) tab.add(evaluated ? mem[a] : -1, fo[a], bad);
-        // per-atom tallies (ev_tally_mb's equal shares): members 1.. by exact
-        // atomics, the owner by runs of equal owners over the wavefront
-        if (A.Eacc || A.Vacc) {
-            if (evaluated)
-#pragma unroll
-                for (int a = 1; a < NB; a++) {
-                    if (A.Eacc) fx_atomic(A.Eacc + 2L * mem[a], Ec / NB, bad);
-                    if (A.Vacc)
-                        for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * mem[a] + k), v[k] / NB, bad);
-                }
-            const int key = evaluated ? mem[0] : -1;
-            if (__ballot(key >= 0)) {
-                const int seg = fx_run_first<64>(key);
-                const int l = threadIdx.x & 63;
-                const int knext = __shfl_down(key, 1, 64);
-                const bool last = key >= 0 && (l == 63 || knext != key);
-                const long o = key >= 0 ? key : 0;
-                if (A.Eacc) lmp_run_add(key, seg, last, Ec / NB, A.Eacc + 2L * o, bad);
-                if (A.Vacc)
-                    for (int k = 0; k < 6; k++) lmp_run_add(key, seg, last, v[k] / NB, A.Vacc + 2L * (6L * o + k), bad);
-            }
-        }
-        // global energy and virial: only their sum over all atoms' words is
-        // read, so the wavefront's totals (fourteen integer parts summed at
-        // once) are added to the words of its first evaluated cluster's owner
-        if (A.Gacc) {
-            const unsigned long long on = __ballot(evaluated);
-            if (on) {
-                const int k0 = __builtin_amdgcn_readlane(mem[0], __ffsll((long long)on) - 1);
-                long long x[16];
-#pragma unroll
-                for (int k = 0; k < 16; k++) x[k] = 0;
-                if (evaluated) {
-                    if (A.eflag_global) fx_split(Ec, x[0], x[1], bad);
-                    if (A.vflag_global)
-#pragma unroll
-                        for (int k = 0; k < 6; k++) fx_split(v[k], x[2 + 2 * k], x[3 + 2 * k], bad);
-                }
-                const long long t = fx_wave_sums16(x);
-                const int l = threadIdx.x & 63;
-                if (l < 14 && t) atomicAdd(A.Gacc + 14L * k0 + l, (unsigned long long)t);
-            }
-        }
+        for (int a = 0; a < NB; a++) tab.add(evaluated ? mem[a] : -1, fo[a], e, vs, A, bad);
+        lmp_global_add(A, evaluated, Ec, v, blockIdx.x & (CHX_LMP_GSLOTS - 1), bad);
         __syncthreads();
-        tab.flush(A.Facc);
+        tab.flush(A);
         __syncthreads();
     }
     if (bad) atomicOr(&A.status[CHX_LMP_ST_FLAGS], CHX_LMP_BAD_RANGE);
 }
 
 // ---------------------------------------------------------------------------
-// Accumulators -> doubles: one thread per atom; block 0 also sums the global
-// energy and virial over the owner atoms (integer sums, exact).
+// Accumulators -> doubles: one thread per atom; block 0 first sums the
+// CHX_LMP_GSLOTS copies of the global energy and virial, one per thread
+// (integer sums, exact).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_lmp_out(chx_lmp_args A, double *F, double *eatom, double *vatom)
+__global__ __launch_bounds__(256) void k_lmp_out(chx_lmp_args A, double *F, double *eatom, double *vatom,
+                                                 double *glob)
 {
+    static_assert(CHX_LMP_GSLOTS == 256, "one copy per thread");
+    if (A.Gacc && blockIdx.x == 0) {
+        __shared__ long long part[4][16];
+        long long x[16];
+        const unsigned long long *g = A.Gacc + 16L * threadIdx.x;
+#pragma unroll
+        for (int k = 0; k < 7; k++) {
+            fx_sum t;
+            t.add(g + 2 * k);
+            x[2 * k] = t.hi;
+            x[2 * k + 1] = t.lo;
+        }
+        x[14] = x[15] = 0;
+        const long long t = fx_wave_sums16(x);
+        const int l = threadIdx.x & 63;
+        if (l < 16) part[threadIdx.x >> 6][l] = t;
+        __syncthreads();
+        if (threadIdx.x < 7) {
+            fx_sum r;
+            for (int w = 0; w < 4; w++) {
+                r.hi += part[w][2 * threadIdx.x];
+                r.lo += part[w][2 * threadIdx.x + 1];
+            }
+            glob[threadIdx.x] = r.value();
+        }
+    }
     const long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= A.nall) return;
     for (int k = 0; k < 3; k++) {
@@ -569,53 +672,6 @@ __global__ __launch_bounds__(256) void k_lmp_out(chx_lmp_args A, double *F, doub
             t.add(A.Vacc + 2 * (6 * a + k));
             vatom[6 * a + k] = t.value();
         }
-}
-
-// global energy and virial: each block sums a strided share of the owner
-// atoms' words (integer sums, exact) and adds them into gsum[7][2]; the
-// last block to finish converts them
-__global__ __launch_bounds__(256) void k_lmp_global(chx_lmp_args A, unsigned long long *gsum, int *done, double *glob)
-{
-    __shared__ long long sh[256], sl[256];
-    __shared__ bool is_last;
-    const long stride = (long)gridDim.x * 256;
-    for (int k = 0; k < 7; k++) {
-        long long hi = 0, lo = 0;
-        for (long a = (long)blockIdx.x * 256 + threadIdx.x; a < A.nall; a += stride) {
-            const unsigned long long *g = A.Gacc + 2 * (7 * a + k);
-            hi += (long long)g[0] + ((long long)g[1] >> 40);
-            lo += (long long)(g[1] & 0xffffffffffull);
-        }
-        sh[threadIdx.x] = hi;
-        sl[threadIdx.x] = lo;
-        __syncthreads();
-        for (int w = 128; w >= 1; w >>= 1) {
-            if ((int)threadIdx.x < w) {
-                sh[threadIdx.x] += sh[threadIdx.x + w];
-                sl[threadIdx.x] += sl[threadIdx.x + w];
-            }
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) {
-            if (sh[0]) atomicAdd(gsum + 2 * k, (unsigned long long)sh[0]);
-            if (sl[0]) atomicAdd(gsum + 2 * k + 1, (unsigned long long)sl[0]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        __threadfence();
-        is_last = atomicAdd(done, 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (is_last && threadIdx.x < 7) {
-        __threadfence();
-        const unsigned long long h = __atomic_load_n(gsum + 2 * threadIdx.x, __ATOMIC_RELAXED);
-        const unsigned long long l = __atomic_load_n(gsum + 2 * threadIdx.x + 1, __ATOMIC_RELAXED);
-        fx_sum t;
-        t.hi = (long long)h + ((long long)l >> 40);
-        t.lo = (long long)(l & 0xffffffffffull);
-        glob[threadIdx.x] = t.value();
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -717,9 +773,10 @@ void launch_lmp_fp_rows(int nb, int mode, long n, const int *list, const chx_lmp
 void launch_lmp_pair(const chx_lmp_args &A, const chx_model_dev &M, const chx_tabs_dev *T, hipStream_t st)
 {
     if (A.inum <= 0) return;
-    const dim3 grid((unsigned)((A.inum + 15) / 16)), block(256);
-    if (T && T->ntab2) hipLaunchKernelGGL(k_lmp_pair<true>, grid, block, 0, st, A, M, *T);
-    else hipLaunchKernelGGL(k_lmp_pair<false>, grid, block, 0, st, A, M, chx_tabs_dev{});
+    const dim3 grid((unsigned)((A.inum + 3) / 4)), block(256);
+    const size_t lds = lmp_table::bytes(LMP_PAIR_SLOTS, A.Eacc || A.Vacc ? 20 : 6);
+    if (T && T->ntab2) hipLaunchKernelGGL(k_lmp_pair<true>, grid, block, lds, st, A, M, *T);
+    else hipLaunchKernelGGL(k_lmp_pair<false>, grid, block, lds, st, A, M, chx_tabs_dev{});
 }
 
 void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, double pad3, double pad4, int has4, int *cnt3,
@@ -752,35 +809,32 @@ void launch_lmp_clusters(int nb, int D, long n, const int *list, double rc, int 
     // two workgroups for each of the 1024 the device holds at once (two
     // wavefronts on each of a CU's SIMDs), fewer for short lists
     const dim3 grid((unsigned)std::min<long>((n + 127) / 128, 2048)), block(128);
+    const size_t lds = lmp_table::bytes(LMP_TILE_SLOTS, A.Eacc || A.Vacc ? 20 : 6);
     if (nb == 3 && T && T->ntab3) {
-        hipLaunchKernelGGL((k_lmp_clusters<3, 0, true>), grid, block, 0, st, count, near, list, A, M, *T);
+        hipLaunchKernelGGL((k_lmp_clusters<3, 0, true>), grid, block, lds, st, count, near, list, A, M, *T);
         return;
     }
 #define X(d)                                                                                                  \
     if (D == d) {                                                                                             \
-        hipLaunchKernelGGL((k_lmp_clusters<3, d, false>), grid, block, 0, st, count, near, list, A, M, chx_tabs_dev{}); \
+        hipLaunchKernelGGL((k_lmp_clusters<3, d, false>), grid, block, lds, st, count, near, list, A, M, chx_tabs_dev{}); \
         return;                                                                                               \
     }
     if (nb == 3) { CHX_D3_CASES(X) }
 #undef X
 #define X(d)                                                                                                  \
     if (D == d) {                                                                                             \
-        hipLaunchKernelGGL((k_lmp_clusters<4, d, false>), grid, block, 0, st, count, near, list, A, M, chx_tabs_dev{}); \
+        hipLaunchKernelGGL((k_lmp_clusters<4, d, false>), grid, block, lds, st, count, near, list, A, M, chx_tabs_dev{}); \
         return;                                                                                               \
     }
     if (nb == 4) { CHX_D4_CASES(X) }
 #undef X
 }
 
-void launch_lmp_out(const chx_lmp_args &A, double *F, double *eatom, double *vatom, double *glob,
-                    unsigned long long *gsum, int *done, hipStream_t st)
+void launch_lmp_out(const chx_lmp_args &A, double *F, double *eatom, double *vatom, double *glob, hipStream_t st)
 {
     if (A.nall > 0)
-        hipLaunchKernelGGL(k_lmp_out, dim3((unsigned)((A.nall + 255) / 256)), dim3(256), 0, st, A, F, eatom, vatom);
-    if (A.Gacc) {
-        const unsigned nb = (unsigned)std::min<long>(256, std::max<long>(1, ((long)A.nall + 1023) / 1024));
-        hipLaunchKernelGGL(k_lmp_global, dim3(nb), dim3(256), 0, st, A, gsum, done, glob);
-    }
+        hipLaunchKernelGGL(k_lmp_out, dim3((unsigned)((A.nall + 255) / 256)), dim3(256), 0, st, A, F, eatom, vatom,
+                           glob);
 }
 
 }  // namespace chx

@@ -37,3 +37,30 @@ def test_rows(tmp_path, natoms, rc4):
     assert np.array_equal(g3, trips) and np.array_equal(g4, quads), (len(trips), len(quads))
     P.close()
     model.close()
+
+
+@pytest.mark.parametrize("natoms", [2, 64, 65, 66, 129, 300])
+def test_pair_rows(tmp_path, natoms):
+    """1-/2-body forces and every tally of owners with up to natoms - 1
+    partners: the queue's batches of 64 and, past 256 atoms, contributions that
+    find the workgroup's table full.  Tolerance: the same FP64 terms on both
+    sides, a few ulp of rounding each, so 1e-10 of the largest component."""
+    from chimes_calculator_amd import GpuModel, LmpPair
+    m = W.Model("ball2", ["C"], (6, 0, 0), (5.0, 0.0, 0.0), {frozenset(("C",)): 0.05}, seed=natoms)
+    pf = m.write(str(tmp_path / "ball2.txt"))
+    rng = np.random.default_rng(natoms)
+    v = rng.normal(size=(natoms, 3))
+    x = 10.0 + v / np.linalg.norm(v, axis=1)[:, None] * 2.4 * rng.random((natoms, 1)) ** (1.0 / 3.0)
+    O = LmpOracle(pf)
+    S = LmpSystem(x, np.ones(natoms, np.int32), rng.permutation(natoms).astype(np.int32) + 1, np.zeros(3),
+                  np.full(3, 20.0), [0], O.rc2(), 1.0, shuffle_seed=1)
+    R = O.compute(S, np.zeros((0, 3), np.int32), np.zeros((0, 4), np.int32))
+    model = GpuModel(pf)
+    P = LmpPair(model, {1: W.MASS["C"]})
+    out = P.compute(S.x, S.type, S.tag, S.ilist, S.numneigh, S.nbr_off, S.nbr, ago=0, skin=1.0)
+    for name, got, ref in zip(("f", "eng", "virial", "eatom", "vatom"), out,
+                              (R.f, R.eng, R.virial, R.eatom, R.vatom)):
+        got, ref = np.asarray(got, float), np.asarray(ref, float)
+        assert np.abs(got - ref).max() <= 1e-10 * max(np.abs(ref).max(), 1e-300), name
+    P.close()
+    model.close()
