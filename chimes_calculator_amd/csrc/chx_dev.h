@@ -261,12 +261,17 @@ __device__ __forceinline__ void fx_cfg_sums(unsigned long long *Cacc, int key, i
 // Per-workgroup LDS table that merges the force contributions of a tile by
 // atom before they reach global memory: open addressing on the atom index,
 // exact integer LDS atomics, then one global atomic pair per component and
-// distinct atom.  CAP must exceed the number of contributions per flush.
+// distinct atom.  An atom's six words lie in one 64-byte line of the
+// accumulator (CHX_FACC_STRIDE) and are added by neighbouring lanes of one
+// instruction, which reach memory as one transaction; a lane per atom adding
+// word after word made six of them.  C/O batch of 4096 configurations: the
+// 3-body kernel 1.78 -> 1.60 ms, the FP32-mixed plan 5.86 -> 5.56 ms.
 template <int CAP>
 struct fx_table {
-    static_assert((CAP & (CAP - 1)) == 0, "table capacity must be a power of two");
+    static_assert((CAP & (CAP - 1)) == 0 && CAP >= 64, "table capacity must be a power of two");
     int key[CAP];
     unsigned long long val[CAP][6];  // (hi, lo) per component
+    unsigned short used[CAP];        // flush: the occupied slots of each 64-slot chunk
 
     // all threads of the block; a barrier must follow before use
     __device__ __forceinline__ void clear()
@@ -277,28 +282,9 @@ struct fx_table {
             for (int k = 0; k < 6; k++) val[s][k] = 0ull;
         }
     }
-    __device__ __forceinline__ void add(int atom, const double (&v)[3], bool &bad)
-    {
-        if (atom < 0) return;
-        unsigned h = ((unsigned)atom * 2654435761u) >> 8;
-        int s = (int)(h & (CAP - 1));
-        for (int probe = 0; probe < CAP; probe++) {
-            const int prev = atomicCAS(&key[s], -1, atom);
-            if (prev == -1 || prev == atom) break;
-            s = (s + 1) & (CAP - 1);
-        }
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            if (v[k] == 0.0) continue;
-            long long hi, lo;
-            fx_split(v[k], hi, lo, bad);
-            if (hi) atomicAdd(&val[s][2 * k], (unsigned long long)hi);
-            if (lo) atomicAdd(&val[s][2 * k + 1], (unsigned long long)lo);
-        }
-    }
-    // as add, but when every slot is taken by other atoms the contribution
-    // goes straight to the global accumulators acc[(3*atom + k)*2 + {0,1}]
-    __device__ __forceinline__ void add_or_global(int atom, const double (&v)[3], unsigned long long *acc, bool &bad)
+    // adds v to the atom's slot; when every slot is taken by other atoms the
+    // contribution goes straight to its words of acc
+    __device__ __forceinline__ void add(int atom, const double (&v)[3], unsigned long long *acc, bool &bad)
     {
         if (atom < 0) return;
         unsigned h = ((unsigned)atom * 2654435761u) >> 8;
@@ -312,22 +298,30 @@ struct fx_table {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             if (v[k] == 0.0) continue;
-            if (!found) { fx_atomic(acc + 2L * (3L * atom + k), v[k], bad); continue; }
+            if (!found) { fx_atomic(acc + (long)CHX_FACC_STRIDE * atom + 2 * k, v[k], bad); continue; }
             long long hi, lo;
             fx_split(v[k], hi, lo, bad);
             if (hi) atomicAdd(&val[s][2 * k], (unsigned long long)hi);
             if (lo) atomicAdd(&val[s][2 * k + 1], (unsigned long long)lo);
         }
     }
-    // all threads of the block, after a barrier
+    // all threads of the block (whole wavefronts), after a barrier
     __device__ __forceinline__ void flush(unsigned long long *acc)
     {
-        for (int s = threadIdx.x; s < CAP; s += blockDim.x) {
-            const int a = key[s];
-            if (a < 0) continue;
-#pragma unroll
-            for (int k = 0; k < 6; k++)
-                if (val[s][k]) atomicAdd(acc + 6L * a + k, val[s][k]);
+        const int lane = threadIdx.x & 63, k = lane & 7;
+        const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+        for (int c = threadIdx.x - lane; c < CAP; c += blockDim.x) {
+            const bool on = key[c + lane] >= 0;
+            const unsigned long long b = __ballot(on);
+            if (on) used[c + __popcll(b & below)] = (unsigned short)(c + lane);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int n = __popcll(b);
+            for (int i = lane >> 3; i < n; i += 8) {
+                const int s = used[c + i];
+                const unsigned long long w = k < 6 ? val[s][k] : 0ull;
+                if (w) atomicAdd(acc + (long)CHX_FACC_STRIDE * key[s] + k, w);
+            }
         }
     }
 };

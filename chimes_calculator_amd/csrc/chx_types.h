@@ -18,6 +18,10 @@
 #define CHX_MFMA3_MAX_D 13     // 3-body dense dimension handled by the matrix-core kernel
 #define CHX_MFMA3V_MAX_D 10    // 3-body dense dimension of the one-cluster-per-lane matrix-core kernel (FP32)
 #define CHX_STATIC_MAX_CLUSTERS 131072  // clusters per call of the allocation-free explicit-cluster entry
+// Force accumulator words per replicated atom: three (hi, lo) pairs and two
+// unused words, one 64-byte line, so that an atom's six atomics are one
+// transaction.
+#define CHX_FACC_STRIDE 8
 // Per-configuration energy and virial accumulators: CHX_CACC_SLOTS copies per
 // configuration, one 128-byte line each (7 (hi, lo) pairs), picked by
 // workgroup, so the wavefronts of one large configuration spread their

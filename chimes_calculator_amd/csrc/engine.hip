@@ -1113,7 +1113,7 @@ void layout(chx_engine *e, const chx_batch *b, bool host_out)
     e->ge3.ensure(G3 + 1);
     e->gb4.ensure(G4 + 1);
     e->ge4.ensure(G4 + 1);
-    e->Facc.ensure(6 * N);
+    e->Facc.ensure(CHX_FACC_STRIDE * N);
     e->Cacc.ensure((long)CHX_CACC_SLOTS * CHX_CACC_STRIDE * ncfg);
     e->part.ensure(14L * e->nitems);
     e->done.ensure(ncfg + 1);
@@ -1209,7 +1209,7 @@ void size_work(chx_engine *e)
     cl[n++] = chx_clear_range{e->cell_cur.p, (long)e->ncell + 1};
     cl[n++] = chx_clear_range{e->cnt34.p, (long)(e->G3 + e->G4) * N + 1};
     if (e->G3 + e->G4) cl[n++] = chx_clear_range{e->nrec.p, N};
-    cl[n++] = chx_clear_range{(int *)e->Facc.p, 12 * N};
+    cl[n++] = chx_clear_range{(int *)e->Facc.p, 2 * CHX_FACC_STRIDE * N};
     cl[n++] = chx_clear_range{(int *)e->Cacc.p, 2L * CHX_CACC_SLOTS * CHX_CACC_STRIDE * e->ncfg};
     cl[n++] = chx_clear_range{e->done.p, (long)e->ncfg + 1};
     e->nclear = n;

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(LPO * OWN) __attribute__((amdgpu_waves_per_eu(3))) 
             auto add = [&](const chx_entry_s &g, double E, double fs, const double (&dr)[3]) {
                 const double F0[3] = {fs * dr[0], fs * dr[1], fs * dr[2]};
                 const double F1[3] = {-F0[0], -F0[1], -F0[2]};
-                tab.add_or_global(g.parent, F1, Facc, bad);
+                tab.add(g.parent, F1, Facc, bad);
                 acc[0] += F0[0];
                 acc[1] += F0[1];
                 acc[2] += F0[2];
@@ -176,9 +176,8 @@ __global__ __launch_bounds__(LPO * OWN) __attribute__((amdgpu_waves_per_eu(3))) 
     // (inclusive sums by row shifts: the owner's last lane holds the total)
 #pragma unroll
     for (int k = 0; k < 10; k++) acc[k] = group_sum<LPO>(acc[k]);
-    if (sub == LPO - 1 && i < natoms)
-#pragma unroll
-        for (int k = 0; k < 3; k++) fx_atomic(Facc + 2L * (3L * i + k), acc[k], bad);
+    const double Fo[3] = {acc[0], acc[1], acc[2]};
+    tab.add(sub == LPO - 1 && i < natoms ? i : -1, Fo, Facc, bad);
     // energy and virial per configuration, exact over the wavefront's owners
     double q7[7];
 #pragma unroll
@@ -411,7 +410,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 3 && 
     // lanes' LDS atomics cost fewer instructions than six wavefront scans);
     // energy and virial go to the configuration
 #pragma unroll
-    for (int m = 0; m < NB; m++) tab.add_or_global(key[m], Fr[m], Facc, bad);
+    for (int m = 0; m < NB; m++) tab.add(key[m], Fr[m], Facc, bad);
     fx_cfg_sums(Cacc, ckey, blockIdx.x & (CHX_CACC_SLOTS - 1), q7, bad);
     __syncthreads();
     tab.flush(Facc);
@@ -913,7 +912,7 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_eval4m(int G, const int *__rest
         for (int w = 16; w <= 32; w <<= 1)
 #pragma unroll
             for (int k = 0; k < 7; k++) q7[k] += __shfl_xor(q7[k], w, 64);
-        st.tab.add(act ? key_s : -1, F, bad);
+        st.tab.add(act ? key_s : -1, F, Facc, bad);
         fx_cfg_sums(Cacc, (act && sub == 0) ? cfg : -1, blockIdx.x & (CHX_CACC_SLOTS - 1), q7, bad);
         __syncthreads();
         st.tab.flush(Facc);
@@ -1152,7 +1151,7 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_eval3m(int G, const int *__rest
     for (int w = 16; w <= 32; w <<= 1)
 #pragma unroll
         for (int k = 0; k < 7; k++) q7[k] += __shfl_xor(q7[k], w, 64);
-    st.tab.add((act && sub < 3) ? key_s : -1, F, bad);
+    st.tab.add((act && sub < 3) ? key_s : -1, F, Facc, bad);
     fx_cfg_sums(Cacc, (act && sub == 0) ? cfg : -1, blockIdx.x & (CHX_CACC_SLOTS - 1), q7, bad);
     __syncthreads();
     st.tab.flush(Facc);
@@ -1348,7 +1347,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         note_flags(cfg_stat, cfg, flags);
     }
 #pragma unroll
-    for (int m = 0; m < NB; m++) sh.tab.add(key[m], Fr[m], bad);
+    for (int m = 0; m < NB; m++) sh.tab.add(key[m], Fr[m], Facc, bad);
     fx_cfg_sums(Cacc, ckey, blockIdx.x & (CHX_CACC_SLOTS - 1), q7, bad);
     __syncthreads();
     sh.tab.flush(Facc);
@@ -1387,7 +1386,7 @@ __global__ __launch_bounds__(256) void k_fin(int ncfg, int nitems, const int *__
         for (int rho = 0; rho < ncopy; rho++) {
             const long r = C.atom_off + (long)rho * C.natoms_in + la;
 #pragma unroll
-            for (int k = 0; k < 3; k++) f[k].add(Facc + 2L * (3L * r + k));
+            for (int k = 0; k < 3; k++) f[k].add(Facc + (long)CHX_FACC_STRIDE * r + 2 * k);
         }
 #pragma unroll
         for (int k = 0; k < 3; k++) Fout[3L * a + k] = f[k].value();
