@@ -317,7 +317,8 @@ def c1_form(args, cpu=False, precision=None):
     # counters of the chosen 4-body kernel from the committed summaries
     v4 = vv[1]
     k4 = ("k_eval4m<%d,%s,%d,0>" % (order4, "double" if prec == cc.FP64 else "float", 4 if v4 == 0 else 2)
-          if v4 in (0, 1) and order4 <= 4 else "k_evalv<4,%d,%s>" % (order4, "double" if prec == cc.FP64 else "float"))
+          if v4 in (0, 1) and order4 <= 4 else "k_lane<4,%d>" % order4 if prec != cc.FP64 and order4 <= 4
+          else "k_evalv<4,%d,%s>" % (order4, "double" if prec == cc.FP64 else "float"))
     prof4 = "k_eval4m_water1536_%s.md" % ("fp64_traffic" if prec == cc.FP64 else "mixed_counters")
     figs4 = profile_figures(prof4, k4)
     out = {
@@ -583,12 +584,12 @@ def bench_c2(args):
     body = 3 if kt["3body"] >= kt["4body"] else 4
     var = variants[body - 3]
     f32 = head_prec == cc.MIXED
-    if var == 2 or (body == 4 and d4 > 4) or (var == 3 and (body == 4 or not f32 or d3 > 10)):
+    if f32 and var >= 2 and (body == 3 or d4 <= 4):
+        kname = "k_lane<%d, %d>" % (body, d3 if body == 3 else d4)
+        unit = "matrix cores and vector ALU (one cluster per lane)"
+    elif var >= 2 or (body == 4 and d4 > 4):
         kname = "k_evalv<%d, %d, %s>" % (body, d3 if body == 3 else d4, "float" if f32 else "double")
         unit = "vector ALU"
-    elif var == 3:
-        kname = "k_eval3v<%d>" % d3
-        unit = "matrix cores (one cluster per lane)"
     else:
         kname = "%s<%d, %s, %d, 0>" % ("k_eval3m" if body == 3 else "k_eval4m", d3 if body == 3 else d4,
                                        "float" if f32 else "double", 4 if var == 0 else 2)

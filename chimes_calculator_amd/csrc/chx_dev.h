@@ -17,6 +17,19 @@ namespace chx {
 
 #define CHX_FX_LIMIT 0x1p42
 
+// Data that earlier kernels wrote and a launch only reads, at a
+// workgroup-uniform index, read through the constant address space: scalar
+// loads into scalar registers.
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T *p, long k)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return ((const __attribute__((address_space(4))) T *)p)[k];
+#else
+    return p[k];  // the host pass never runs device code
+#endif
+}
+
 // Status flags as one value for the whole workgroup (read once, then shared),
 // so that every wave of a block takes the same early exit.
 __device__ __forceinline__ bool block_stop(const int *status, int mask)
@@ -282,15 +295,15 @@ struct fx_table {
             for (int k = 0; k < 6; k++) val[s][k] = 0ull;
         }
     }
-    // adds v to the atom's slot; when every slot is taken by other atoms the
-    // contribution goes straight to its words of acc
+    // adds v to the atom's slot; an atom that finds none within sixteen
+    // probes has its contribution go straight to its words of acc
     __device__ __forceinline__ void add(int atom, const double (&v)[3], unsigned long long *acc, bool &bad)
     {
         if (atom < 0) return;
         unsigned h = ((unsigned)atom * 2654435761u) >> 8;
         int s = (int)(h & (CAP - 1));
         bool found = false;
-        for (int probe = 0; probe < CAP; probe++) {
+        for (int probe = 0; probe < 16; probe++) {
             const int prev = atomicCAS(&key[s], -1, atom);
             if (prev == -1 || prev == atom) { found = true; break; }
             s = (s + 1) & (CAP - 1);

@@ -37,16 +37,15 @@ bool supported_D4(int D);
 void launch_eval2(int natoms, int nb_cap, hipStream_t st, const int *nbr_cnt, const chx_cfg *cfgs,
                   const chx_atom_s *as, const chx_entry_s *es, const chx_model_dev *models, unsigned long long *Facc,
                   unsigned long long *Cacc, int *cfg_stat, int *status);
-// Vector-unit kernel for nb = 3 or 4 bodies.
+// One-cluster-per-lane kernels for nb = 3 or 4 bodies.
 void launch_evalv(int nb, int D, int prec, const chx_list_args &la, hipStream_t st);
 // nb-body evaluation at precision prec (chx_precision) with the given kernel
-// variant (CHX_VAR_*; BF16 always uses the matrix cores); the vector kernel
-// (FP32 for the reduced precisions) stands in where the matrix-core kernels
-// do not take D.
+// variant (CHX_VAR_*; BF16 always uses the matrix cores); the
+// one-cluster-per-lane kernel (FP32 for the reduced precisions) stands in
+// where the matrix-core kernels do not take D.
 void launch_eval_body(int nb, int D, int prec, int variant, const chx_list_args &la, hipStream_t st);
-// Whether variant has a kernel of its own for nb bodies at precision prec
-// (the one-cluster-per-lane matrix-core variant: 3-body FP32-mixed only).
-bool variant_applies(int nb, int prec, int variant);
+// Whether variant names a kernel of its own (CHX_VAR_MFMAV is CHX_VAR_VECTOR's).
+bool variant_applies(int variant);
 void launch_clusters(int nb, int D, int n, hipStream_t st, const double *dist, const double *drv, const int *types,
                      const chx_model_dev &M, double *E, double *F, double *S, double *last, int *flags);
 

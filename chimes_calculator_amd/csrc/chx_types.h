@@ -16,7 +16,6 @@
 #define CHX_LIST_ALIGN 64      // 3-/4-body list segments of one cluster type start on this multiple
 #define CHX_MFMA_MAX_D 4       // 4-body dense dimension handled by the matrix-core kernel
 #define CHX_MFMA3_MAX_D 13     // 3-body dense dimension handled by the matrix-core kernel
-#define CHX_MFMA3V_MAX_D 10    // 3-body dense dimension of the one-cluster-per-lane matrix-core kernel (FP32)
 #define CHX_STATIC_MAX_CLUSTERS 131072  // clusters per call of the allocation-free explicit-cluster entry
 // Force accumulator words per replicated atom: three (hi, lo) pairs and two
 // unused words, one 64-byte line, so that an atom's six atomics are one
@@ -63,9 +62,10 @@ struct chx_clear_range {
 
 // 3-/4-body evaluation kernel variants (chosen per body order by the plan
 // autotuner): matrix cores with 4 or 2 wavefronts per workgroup (64 or 32
-// clusters per tile), the vector units, or (3-body, FP32-mixed) one cluster
-// per lane with the contraction on the matrix cores; where a variant does
-// not apply the vector kernel stands in.
+// clusters per tile), or one cluster per lane: FP64 on the vector units,
+// FP32-mixed with the contraction on the matrix cores (3-body; 4-body D <= 4).
+// CHX_VAR_MFMAV names that FP32-mixed kernel too; where a matrix-core variant
+// does not apply the one-cluster-per-lane kernel stands in.
 enum { CHX_VAR_MFMA4 = 0, CHX_VAR_MFMA2 = 1, CHX_VAR_VECTOR = 2, CHX_VAR_MFMAV = 3, CHX_NVAR = 4 };
 #define CHX_SCAN1_MAX 32768    // scans up to this length run in one workgroup
 
@@ -136,6 +136,7 @@ struct chx_group {
     const int *perm;           // canonical member order per type tuple
     const double *C;           // dense coefficients, parameter pair order
     const float *Cf;           // FP32 copy
+    const float *Cl;           // FP32 image(s) of the one-cluster-per-lane matrix-core kernels (chx_lane.h)
     const double *Cm;          // 4-body matrix image for the matrix-core kernel (D <= 4)
     const float *Cmf;          // FP32 copy
     const unsigned short *Cmb; // BF16 images (rounded, then residual), transposed: [column][row padded to 32]

@@ -33,6 +33,7 @@
 
 #include "chx_engine.h"
 #include "chx_eval.h"
+#include "chx_lane.h"
 #include "chx_kernels.h"
 #include "chx_fp.h"
 #include "chx_lmp.h"
@@ -251,6 +252,7 @@ struct TypeLaunch {
     chx_slot s[6];
     const double *C = nullptr;   // device, FP64 dense coefficients
     const float *Cf = nullptr;   // device, FP32 copy for the mixed path
+    const float *Cl = nullptr;   // device, FP32 image for the one-cluster-per-lane kernels
     const double *Cm = nullptr;  // device, matrix image for the matrix-core kernels
     const float *Cmf = nullptr;
     const unsigned short *Cmb = nullptr;  // device, BF16 images (rounded, residual) transposed [column][row to 32]
@@ -331,6 +333,29 @@ std::vector<double> trip_matrix_image(const double *C, int D)
     for (int a = 0; a < D; a++)
         for (int b = 0; b < D; b++)
             for (int c = 0; c < D; c++) m[(size_t)a * MP + 16 * b + c] = C[((size_t)a * D + b) * D + c];
+    return m;
+}
+
+// Images of the one-cluster-per-lane matrix-core kernels (chx_lane.h).
+std::vector<float> trip_lane_image(const double *C, int D)
+{
+    const int NQ = (D * D + 3) / 4, NV = (NQ * D + 15) / 16;
+    std::vector<float> m((size_t)NV * 64, 0.f);
+    for (int r = 0; r < D * D; r++)
+        for (int k = 0; k < D; k++) m[((size_t)(r / 4) * D + k) * 4 + r % 4] = (float)C[(size_t)r * D + k];
+    return m;
+}
+
+std::vector<float> quad_lane_image(const double *C, int D)
+{
+    const int R = D * D * D, NQ = (R + 3) / 4, NV = (R * NQ + 15) / 16;
+    std::vector<float> m((size_t)2 * NV * 64, 0.f);
+    for (int k = 0; k < R; k++)
+        for (int c = 0; c < R; c++) {
+            const size_t at = ((size_t)(R - 1 - k) * NQ + c / 4) * 4 + c % 4;
+            m[at] = (float)C[(size_t)k * R + c];
+            m[(size_t)NV * 64 + at] = (float)C[(size_t)c * R + k];
+        }
     return m;
 }
 
@@ -684,6 +709,8 @@ chx_model *chx_model_create(chx_engine *e, const chx_model_desc *d)
                 for (int q = 0; q < 3; q++) m->t3[t].s[q] = s3[3 * t + q];
                 m->t3[t].C = v.C3 + t * cs;
                 m->t3[t].Cf = Cf + t * cs;
+                const std::vector<float> imgl = trip_lane_image(d->C3 + t * cs, d->D3);
+                m->t3[t].Cl = m->up(imgl.data(), imgl.size());
                 if (d->D3 <= CHX_MFMA3_MAX_D) {
                     const std::vector<double> img = trip_matrix_image(d->C3 + t * cs, d->D3);
                     const std::vector<float> imgf(img.begin(), img.end());
@@ -718,6 +745,10 @@ chx_model *chx_model_create(chx_engine *e, const chx_model_desc *d)
                 for (int q = 0; q < 6; q++) m->t4[t].s[q] = s4[6 * t + q];
                 m->t4[t].C = v.C4 + t * cs;
                 m->t4[t].Cf = Cf + t * cs;
+                if (d->D4 <= CHX_LANE4_MAX_D) {
+                    const std::vector<float> imgl = quad_lane_image(d->C4 + t * cs, d->D4);
+                    m->t4[t].Cl = m->up(imgl.data(), imgl.size());
+                }
                 if (d->D4 <= CHX_MFMA_MAX_D) {
                     const std::vector<double> img = quad_matrix_image(d->C4 + t * cs, d->D4);
                     const std::vector<float> imgf(img.begin(), img.end());
@@ -1067,6 +1098,7 @@ void prepare(chx_engine *e, chx_model *const *models, int nmodels, const chx_bat
                     const TypeLaunch &tl = body == 3 ? M->t3[t] : M->t4[t];
                     g.C = tl.C;
                     g.Cf = tl.Cf;
+                    g.Cl = tl.Cl;
                     g.Cm = tl.Cm;
                     g.Cmf = tl.Cmf;
                     g.Cmb = tl.Cmb;
@@ -1642,7 +1674,7 @@ void plan_tune(chx_plan *p, chx_out *o)
         // the BF16 forms are defined by their matrix-core contraction: no vector variant
         const int nvar = e->prec >= CHX_BF16 ? CHX_VAR_VECTOR : CHX_NVAR;
         for (int var = 0; var < nvar; var++) {
-            if (!variant_applies(body, e->prec, var)) continue;
+            if (!variant_applies(var)) continue;
             float best_rep = 1e30f;
             for (int rep = 0; rep < 3; rep++) {
                 HIPCHK(hipEventRecord(a, e->st));
@@ -1679,7 +1711,7 @@ void plan_tune(chx_plan *p, chx_out *o)
         const int nvar = prec >= CHX_BF16 ? CHX_VAR_VECTOR : CHX_NVAR;
         std::vector<int> order;
         for (int v = 0; v < nvar; v++)
-            if (variant_applies(body, prec, v)) order.push_back(v);
+            if (variant_applies(v)) order.push_back(v);
         std::stable_sort(order.begin(), order.end(),
                          [&](int x, int y) { return p->tune_ms[body - 3][x] < p->tune_ms[body - 3][y]; });
         int chosen = -1;

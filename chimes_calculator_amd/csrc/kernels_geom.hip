@@ -666,19 +666,6 @@ __device__ __forceinline__ void enum_queue_big(const chx_enum_args &x, int i)
     if (!x.big_on) atomicOr(&x.status[CHX_ST_FLAGS], CHX_RETRY_BIG);
 }
 
-// Data that earlier kernels wrote and a launch only reads, at a
-// workgroup-uniform index, read through the constant address space: scalar
-// loads into scalar registers.
-template <typename T>
-__device__ __forceinline__ T uniform_load(const T *p, long k)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    return ((const __attribute__((address_space(4))) T *)p)[k];
-#else
-    return p[k];  // the host pass never runs device code
-#endif
-}
-
 template <int C3, int C4, int NT>
 __device__ __forceinline__ void enum_owner(const chx_enum_args &x, int i, EnumShared<C3, C4> &sh)
 {

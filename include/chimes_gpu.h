@@ -26,8 +26,9 @@ enum { CHIMES_GPU_FP64 = 0, CHIMES_GPU_MIXED = 1, CHIMES_GPU_BF16 = 2, CHIMES_GP
 enum {
     CHIMES_GPU_VAR_MFMA4 = 0,  /* matrix cores, 64-cluster tiles */
     CHIMES_GPU_VAR_MFMA2 = 1,  /* matrix cores, 32-cluster tiles */
-    CHIMES_GPU_VAR_VECTOR = 2, /* vector units, one cluster per lane */
-    CHIMES_GPU_VAR_MFMAV = 3   /* one cluster per lane, 3-body contraction on the matrix cores (FP32-mixed) */
+    CHIMES_GPU_VAR_VECTOR = 2, /* one cluster per lane: vector units; FP32-mixed with the contraction on the
+                                  matrix cores (4-body: D <= 4) */
+    CHIMES_GPU_VAR_MFMAV = 3   /* as CHIMES_GPU_VAR_VECTOR */
 };
 
 /* Parses a ChIMES parameter file and uploads its tables to GPU `device`. */
@@ -93,9 +94,8 @@ chimes_gpu_plan *chimes_gpu_plan_create_device(chimes_gpu_model *const *models, 
 int chimes_gpu_plan_run_device(chimes_gpu_plan *p, const double *cells, double *energy_dev, double *forces_dev,
                                double *virial_dev);
 /* variants[2]: kernel variant of the 3- and 4-body terms (0 matrix cores,
- * 64-cluster tiles; 1 matrix cores, 32-cluster tiles; 2 vector units; 3 one
- * cluster per lane with the contraction on the matrix cores, 3-body
- * FP32-mixed only, D <= 10);
+ * 64-cluster tiles; 1 matrix cores, 32-cluster tiles; 2 and 3 one cluster per
+ * lane, timed as 2);
  * tune_ms[8]: timed milliseconds per (body, variant), tune_ms[4 (body - 3) +
  * variant], 0 if not tuned or not applicable, negated
  * for a variant the tuner rejected: the tuner keeps the fastest variant whose
@@ -109,13 +109,13 @@ void chimes_gpu_plan_free(chimes_gpu_plan *p);
  * chimes_gpu_plan_info; -1 keeps the current one).  chimes_gpu_set_variants
  * sets them for every later evaluation on `device` that does not go through
  * a plan (chimes_gpu_eval_batch*, calculate_chimes*, the chimesFF classes);
- * the defaults are 2 (vector units) for the 3-body and 0 (matrix cores,
+ * the defaults are 2 (one cluster per lane) for the 3-body and 0 (matrix cores,
  * 64-cluster tiles) for the 4-body term.  chimes_gpu_plan_set_variants sets
  * them for a plan, whose next run evaluates directly and captures again.  A
  * matrix-core variant for a dense dimension above the matrix-core kernels'
- * range (4-body D > 4) runs on the vector units, and so does variant 3 where
- * it does not apply (4-body, FP64, 3-body D > 10); a vector-unit request of a
- * BF16 form runs on the matrix cores.  Nonzero for an unknown variant. */
+ * range (4-body D > 4) runs with one cluster per lane; a one-cluster-per-lane
+ * request of a BF16 form runs on the matrix cores.  Nonzero for an unknown
+ * variant. */
 int chimes_gpu_set_variants(int device, int var3, int var4);
 int chimes_gpu_get_variants(int device, int variants[2]);
 int chimes_gpu_plan_set_variants(chimes_gpu_plan *p, int var3, int var4);
