@@ -66,6 +66,36 @@ __device__ __forceinline__ void fx_split(double v, long long &hi, long long &lo,
     lo = (long long)((s - f) * 0x1p40);
 }
 
+// The splits of N contributions, hi and lo of each in turn in p: one range test
+// for all of them.
+template <int N>
+__device__ __forceinline__ void fx_split_n(const double (&v)[N], long long (&p)[2 * N], bool &bad)
+{
+    bool in = fabs(v[0]) < 0x1p31;
+#pragma unroll
+    for (int k = 1; k < N; k++) in = in && fabs(v[k]) < 0x1p31;
+    if (in) {
+        const double M = 0x1.8p52;
+#pragma unroll
+        for (int k = 0; k < N; k++) {  // as in fx_split
+            const double s = v[k] * 0x1p20, t = s + M, r = s - (t - M);
+            p[2 * k] = __double_as_longlong(t) - __double_as_longlong(M);
+            p[2 * k + 1] = __double_as_longlong(fma(r, 0x1p40, M)) - __double_as_longlong(M);
+        }
+    } else {
+        // rare: one copy of the general split in a loop, so that it does not
+        // take N times its code from the instruction cache
+        double tv[N];
+        long long tp[2 * N];
+#pragma unroll
+        for (int k = 0; k < N; k++) tv[k] = v[k];
+#pragma unroll 1
+        for (int k = 0; k < N; k++) fx_split(tv[k], tp[2 * k], tp[2 * k + 1], bad);
+#pragma unroll
+        for (int k = 0; k < 2 * N; k++) p[k] = tp[k];
+    }
+}
+
 // acc[0] += hi, acc[1] += lo (integer atomics; zero parts are skipped).
 __device__ __forceinline__ void fx_atomic(unsigned long long *acc, double v, bool &bad)
 {
@@ -243,12 +273,14 @@ __device__ __forceinline__ void fx_cfg_sums(unsigned long long *Cacc, int key, i
     const int k0 = __builtin_amdgcn_readlane(key, __ffsll((long long)act) - 1);
     const int l = threadIdx.x & 63;
     if (__ballot(key >= 0 && key != k0) == 0) {
-        long long x[16];
+        long long x[16], p[14];
+        // every lane's parts, of zeros where it has no cluster
+        double z[7];
 #pragma unroll
-        for (int k = 0; k < 7; k++) {
-            x[2 * k] = x[2 * k + 1] = 0;
-            if (key >= 0) fx_split(q[k], x[2 * k], x[2 * k + 1], bad);
-        }
+        for (int k = 0; k < 7; k++) z[k] = key >= 0 ? q[k] : 0.0;
+        fx_split_n<7>(z, p, bad);
+#pragma unroll
+        for (int k = 0; k < 14; k++) x[k] = p[k];
         x[14] = x[15] = 0;
         const long long t = fx_wave_sums16(x);
         if (l < 14 && t) atomicAdd(fx_cfg_line(Cacc, k0, slot) + l, (unsigned long long)t);
@@ -257,17 +289,19 @@ __device__ __forceinline__ void fx_cfg_sums(unsigned long long *Cacc, int key, i
     const int seg = fx_run_first<64>(key);
     const int knext = __shfl_down(key, 1, 64);
     const bool last = key >= 0 && (l == 63 || knext != key);
+    double tq[7];
 #pragma unroll
-    for (int k = 0; k < 7; k++) {
+    for (int k = 0; k < 7; k++) tq[k] = q[k];
+#pragma unroll 1
+    for (int k = 0; k < 7; k++) {  // a loop: few wavefronts come here, and unrolled it is most of the code
         long long x[2] = {0, 0};
-        if (key >= 0) fx_split(q[k], x[0], x[1], bad);
+        if (key >= 0) fx_split(tq[k], x[0], x[1], bad);
         fx_run_scan<64, 2>(x, seg);
         if (last) {
             unsigned long long *a = fx_cfg_line(Cacc, key, slot) + 2 * k;
             if (x[0]) atomicAdd(a, (unsigned long long)x[0]);
             if (x[1]) atomicAdd(a + 1, (unsigned long long)x[1]);
         }
-        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -308,15 +342,15 @@ struct fx_table {
             if (prev == -1 || prev == atom) { found = true; break; }
             s = (s + 1) & (CAP - 1);
         }
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            if (v[k] == 0.0) continue;
-            if (!found) { fx_atomic(acc + (long)CHX_FACC_STRIDE * atom + 2 * k, v[k], bad); continue; }
-            long long hi, lo;
-            fx_split(v[k], hi, lo, bad);
-            if (hi) atomicAdd(&val[s][2 * k], (unsigned long long)hi);
-            if (lo) atomicAdd(&val[s][2 * k + 1], (unsigned long long)lo);
+        if (!found) {
+            for (int k = 0; k < 3; k++) fx_atomic(acc + (long)CHX_FACC_STRIDE * atom + 2 * k, v[k], bad);
+            return;
         }
+        long long p[6];
+        fx_split_n<3>(v, p, bad);
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+            if (p[k]) atomicAdd(&val[s][k], (unsigned long long)p[k]);  // small forces have no high part
     }
     // all threads of the block (whole wavefronts), after a barrier
     __device__ __forceinline__ void flush(unsigned long long *acc)

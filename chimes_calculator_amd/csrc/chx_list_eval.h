@@ -113,11 +113,11 @@ struct pairs_of<4> {
 };
 
 // Cluster geometry in canonical order: members, pair vectors and distances,
-// and whether every pair is inside its cutoff; canonical member a is runtime
-// member pm[a] (runtime member 0 is the owner).
-template <int NB>
-__device__ __forceinline__ bool cluster_geometry(const chx_group &grp, const int2 rec,
-                                                 const chx_cfg *__restrict__ cfgs,
+// and whether every pair is inside its cutoff (rout(q) of slot q); canonical
+// member a is runtime member pm[a] (runtime member 0 is the owner).
+template <int NB, class ROUT>
+__device__ __forceinline__ bool cluster_geometry(int nt, const int *__restrict__ perm, const ROUT &rout,
+                                                 const int2 rec, const chx_cfg *__restrict__ cfgs,
                                                  const chx_atom_s *__restrict__ as, int nb_cap,
                                                  const chx_entry_s *__restrict__ es, double (&p)[NB][3],
                                                  int (&par)[NB], double (&r)[pairs_of<NB>::P], int &cfg,
@@ -128,16 +128,28 @@ __device__ __forceinline__ bool cluster_geometry(const chx_group &grp, const int
     load_members<NB>(rec, as, nb_cap, es, p, t, par, cfg);
     int tup = 0;
 #pragma unroll
-    for (int a = 0; a < NB; a++) tup = tup * grp.nt + t[a];
-    canonical<NB>(grp.perm, tup, p, par, pm);
+    for (int a = 0; a < NB; a++) tup = tup * nt + t[a];
+    canonical<NB>(perm, tup, p, par, pm);
     const chx_cfg &C = cfgs[cfg];
     bool in = true;
 #pragma unroll
     for (int q = 0; q < PQ::P; q++) {
         r[q] = pair_vec(C.h, p[PQ::a[q]], p[PQ::b[q]], dr[q]);
-        in = in && (r[q] < grp.s[q].rout);
+        in = in && (r[q] < rout(q));
     }
     return in;
+}
+
+template <int NB>
+__device__ __forceinline__ bool cluster_geometry(const chx_group &grp, const int2 rec,
+                                                 const chx_cfg *__restrict__ cfgs,
+                                                 const chx_atom_s *__restrict__ as, int nb_cap,
+                                                 const chx_entry_s *__restrict__ es, double (&p)[NB][3],
+                                                 int (&par)[NB], double (&r)[pairs_of<NB>::P], int &cfg,
+                                                 int (&pm)[NB], double (&dr)[pairs_of<NB>::P][3])
+{
+    return cluster_geometry<NB>(grp.nt, grp.perm, [&](int q) { return grp.s[q].rout; }, rec, cfgs, as, nb_cap, es, p,
+                                par, r, cfg, pm, dr);
 }
 
 // The same without the pair vectors.

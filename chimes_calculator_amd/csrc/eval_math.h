@@ -33,18 +33,20 @@ __device__ __forceinline__ void cheby(double r, const chx_slot &s, R (&T)[D], R 
     const double xd = (ex - s.xavg) * s.ixdiff;
     const double dxdr_d = (-ex * s.ilam) * s.ixdiff;
     const R x = (R)xd, dxdr = (R)dxdr_d, two_x = (R)(2.0 * xd);
-    R U[D];
+    // V_i = U_i dx/dr by the same recurrence, so dT_i/dr = i V_{i-1}; one fused
+    // operation a step
+    R V[D];
     T[0] = (R)1;
-    U[0] = (R)1;
-    if (D > 1) { T[1] = x; U[1] = two_x; }
+    V[0] = dxdr;
+    if (D > 1) { T[1] = x; V[1] = two_x * dxdr; }
 #pragma unroll
     for (int i = 2; i < D; i++) {
-        T[i] = two_x * T[i - 1] - T[i - 2];
-        U[i] = two_x * U[i - 1] - U[i - 2];
+        T[i] = fma(two_x, T[i - 1], -T[i - 2]);
+        V[i] = fma(two_x, V[i - 1], -V[i - 2]);
     }
     dT[0] = (R)0;
 #pragma unroll
-    for (int i = 1; i < D; i++) dT[i] = (R)i * dxdr * U[i - 1];
+    for (int i = 1; i < D; i++) dT[i] = (R)i * V[i - 1];
     if (oor) {
         flags |= FLAG_OUT_OF_RANGE;
         const double damp = exp((r - s.rin) / CHX_SMOOTH);
@@ -99,17 +101,19 @@ __device__ __forceinline__ void eval_pair(double r, const chx_slot &s, const dou
     const double dxdr = (-ex * s.ilam) * s.ixdiff;
     const double two_x = 2.0 * x;
     double Tm2 = 1.0, Tm1 = x, Um2 = 1.0, Um1 = two_x;
-    double sT = c2[1] * x, sdT = c2[1] * dxdr;
+    // sum c_n T_n and sum n c_n U_{n-1}, the latter times dx/dr at the end
+    double sT = c2[1] * x, sdT = c2[1], dn = 1.0;
     for (int n = 2; n <= order; n++) {
-        const double Tn = two_x * Tm1 - Tm2;
-        const double dTn = (double)n * dxdr * Um1;
-        const double Un = two_x * Um1 - Um2;
+        const double Tn = fma(two_x, Tm1, -Tm2);
+        const double Un = fma(two_x, Um1, -Um2);
         const double c = c2[n];
+        dn += 1.0;
         sT = fma(c, Tn, sT);
-        sdT = fma(c, dTn, sdT);
+        sdT = fma(dn * c, Um1, sdT);
         Tm2 = Tm1; Tm1 = Tn;
         Um2 = Um1; Um1 = Un;
     }
+    sdT *= dxdr;
     if (oor) {
         flags |= FLAG_OUT_OF_RANGE;
         const double damp = exp((r - s.rin) / CHX_SMOOTH);

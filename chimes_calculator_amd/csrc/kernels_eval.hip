@@ -42,7 +42,10 @@ typedef float flt4 __attribute__((ext_vector_type(4)));
 // key, and row shifts add the lanes), so the sum depends only on the owner's
 // own images, never on the batch around it; the force is then added exactly
 // per owner, the energy and virial exactly per configuration.  Image forces
-// are merged in the workgroup's LDS table.
+// are merged in the workgroup's LDS table.  Bound by its dependent loads and
+// the accumulation; C/O batch of 4096 configurations (10 M images): 0.47 ms,
+// 0.37 with dx/dr taken out of the Chebyshev loop, the owner's force through
+// the table and no FP64 literals held (and spilled) across the image loop.
 // ---------------------------------------------------------------------------
 template <int OWN, int LPO>
 __global__ __launch_bounds__(LPO * OWN) __attribute__((amdgpu_waves_per_eu(3))) void k_eval2(int natoms, int nb_cap, const int *__restrict__ nbr_cnt,

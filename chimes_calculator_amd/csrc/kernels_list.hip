@@ -64,18 +64,25 @@ __device__ __forceinline__ void lane_contract3(const float (&A)[lane3_shape<D>::
 #pragma unroll
     for (int u = 0; u < D; u++) { t1[u] = T[1][u]; d1[u] = dT[1][u]; }
     double s0 = 0, g00 = 0, g01 = 0, g02 = 0, s1 = 0, g11 = 0, g12 = 0;
-    static_for<SH::NQ>([&](auto Qc) {
-        constexpr int Q = Qc;
-        flt4 z = {0.f, 0.f, 0.f, 0.f}, w = {0.f, 0.f, 0.f, 0.f};
+    // two blocks at a time: four independent chains of matrix instructions
+    static_for<(SH::NQ + 1) / 2>([&](auto Hc) {
+        constexpr int H = 2 * Hc, N = SH::NQ - H < 2 ? 1 : 2;
+        flt4 z[2] = {}, w[2] = {};
         static_for<D>([&](auto Kc) {
-            constexpr int k = Kc, idx = Q * D + k;
-            z = lane_fma4<idx % 16>(A[idx / 16], k == 0 ? 1.f : T[2][k], z);
-            if constexpr (k > 0) w = lane_fma4<idx % 16>(A[idx / 16], dT[2][k], w);
+            constexpr int k = Kc;
+            static_for<N>([&](auto Jc) {
+                constexpr int j = Jc, idx = (H + j) * D + k;
+                z[j] = lane_fma4<idx % 16>(A[idx / 16], k == 0 ? 1.f : T[2][k], z[j]);
+            });
+            static_for<N>([&](auto Jc) {
+                constexpr int j = Jc, idx = (H + j) * D + k;
+                if constexpr (k > 0) w[j] = lane_fma4<idx % 16>(A[idx / 16], dT[2][k], w[j]);
+            });
         });
-        static_for<4>([&](auto Ic) {
-            constexpr int r = 4 * Q + Ic, a0 = r / D, a1 = r % D;
+        static_for<4 * N>([&](auto Ic) {
+            constexpr int r = 4 * H + Ic, a0 = r / D, a1 = r % D;
             if constexpr (r < D * D) {
-                const double zr = z[r % 4], wr = w[r % 4];
+                const double zr = z[Ic / 4][r % 4], wr = w[Ic / 4][r % 4];
                 if constexpr (a1 == 0) {
                     s1 = zr;
                     g11 = 0;
@@ -252,7 +259,8 @@ __device__ __forceinline__ void lane_contract4(const float *__restrict__ img, co
 // consecutive tiles share is flushed once.  C/O batch of 4096 configurations
 // (26.3 M triplets, 13.2 M quadruplets): 3-body D = 7 1.60 ms on the vector
 // ALU, 1.63 ms here with one tile, 1.43 with four, 1.41 with eight; 4-body
-// D = 3 1.33 ms on the vector ALU, 1.27 with four, 1.29 with eight.  Carbon,
+// D = 3 1.33 ms on the vector ALU, 1.27 with four, 1.29 with eight (1.16 since
+// the recurrences and splits were shortened).  Carbon,
 // 32768 atoms: 3-body D = 10 156 -> 129 us, 4-body D = 4 202 -> 167 us.
 //
 // The file is compiled without the hoisting of constants out of that loop
@@ -300,10 +308,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lane_waves<
         if (t0 >= total) break;
         while (g + 1 < G && uniform_load(gbase, g + 1) <= t0) g++;
         g = __builtin_amdgcn_readfirstlane(g);
-        // read through the constant address space: past the first tile's
-        // atomics the compiler would not use scalar loads by itself
-        const chx_group grp = uniform_load(groups, g);
-        if (!(grp.type >= 0 && grp.D == D)) continue;
+        // read through the constant address space, field by field where they
+        // are used: past the first tile's atomics the compiler would not use
+        // scalar loads by itself, and a copy of the whole group spilled
+        // scalar registers
+        const const_ptr<chx_group> grp = (const_ptr<chx_group>)(groups + g);
+        auto slot = [&](int q) {
+            chx_slot s;
+            s.rin = grp->s[q].rin; s.rout = grp->s[q].rout;
+            s.xavg = grp->s[q].xavg; s.ilam = grp->s[q].ilam; s.ixdiff = grp->s[q].ixdiff;
+            s.irout = grp->s[q].irout; s.iramp = grp->s[q].iramp;
+            return s;
+        };
+        if (!(grp->type >= 0 && grp->D == D)) continue;
         const int end = uniform_load(gend, g);
         const long c = t0 + lane;
         int ckey = -1;
@@ -315,11 +332,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lane_waves<
         double p[NB][3], r[P], dr[P][3], S, Gq[P];
         int par[NB], cfg = 0, pm[NB], flags = 0;
         bool act = false;
-        if (c < end) act = cluster_geometry<NB>(grp, list[c], cfgs, as, nb_cap, es, p, par, r, cfg, pm, dr);
+        if (c < end)
+            act = cluster_geometry<NB>(grp->nt, grp->perm, [&](int q) { return grp->s[q].rout; }, list[c], cfgs, as,
+                                       nb_cap, es, p, par, r, cfg, pm, dr);
         auto finish = [&]() {
             double f[P], fd[P], E, fs[P];
 #pragma unroll
-            for (int q = 0; q < P; q++) fcut(r[q], grp.s[q], grp.tersoff, grp.fcut_var, f[q], fd[q]);
+            for (int q = 0; q < P; q++) fcut(r[q], slot(q), grp->tersoff, grp->fcut_var, f[q], fd[q]);
             cluster_scalars<P, double>(r, f, fd, S, Gq, E, fs);
             q7[0] = E;
             cluster_forces<NB>(dr, fs, Fr, q7);
@@ -331,17 +350,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(lane_waves<
         if (__ballot(act) == 0) continue;
         // whole wavefront: lanes without a cluster at the cutoffs
 #pragma unroll
-        for (int q = 0; q < P; q++) r[q] = act ? r[q] : grp.s[q].rout;
+        for (int q = 0; q < P; q++) r[q] = act ? r[q] : grp->s[q].rout;
         float T[P][D], dT[P][D];
 #pragma unroll
-        for (int q = 0; q < P; q++) cheby<D, float>(r[q], grp.s[q], T[q], dT[q], flags);
+        for (int q = 0; q < P; q++) cheby<D, float>(r[q], slot(q), T[q], dT[q], flags);
         if constexpr (NB == 3) {
             float A[lane3_shape<D>::NV];
 #pragma unroll
-            for (int v = 0; v < lane3_shape<D>::NV; v++) A[v] = grp.Cl[64 * v + lane];
+            for (int v = 0; v < lane3_shape<D>::NV; v++) A[v] = grp->Cl[64 * v + lane];
             lane_contract3<D>(A, T, dT, S, Gq);
         } else {
-            lane_contract4<D>(grp.Cl, T, dT, S, Gq);
+            lane_contract4<D>(grp->Cl, T, dT, S, Gq);
         }
         // the folds stay here: moved into the branch below, where their
         // results are used, they would keep every product alive
