@@ -179,8 +179,11 @@ class GpuModel:
         return self.L.chimes_gpu_model_type_index(self.h, name.encode())
 
     def types_to_index(self, types):
-        idx = np.array([self.type_index(t) for t in types], dtype=np.int32)
-        if (idx < 0).any():
+        # one library call per element name, not per atom: a batch of 64
+        # configurations spent 2 of its 2.6 ms in those calls
+        lut = {t: self.type_index(t) for t in set(types)}
+        idx = np.fromiter(map(lut.__getitem__, types), np.int32, len(types))
+        if any(k < 0 for k in lut.values()):
             raise ChimesError("unknown atom type(s): %s" % sorted({t for t, k in zip(types, idx) if k < 0}))
         return idx
 
