@@ -463,16 +463,29 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_eval4m(int G, const int *__rest
             R T2[D], dT2[D];
 #pragma unroll
             for (int x = 0; x < D; x++) { T2[x] = Tj[2 * D + x]; dT2[x] = dTj[2 * D + x]; }
+            // this lane's operand values, the same for every row block
+            R xs[SH::KS], ys[SH::KS];
+#pragma unroll
+            for (int b = 0; b < D; b++) {
+                const R x1 = T1[b] * t2, y1 = T4[b] * t5;
+#pragma unroll
+                for (int a = 0; a < D; a++) {
+                    xs[a * D + b] = T0[a] * x1;
+                    ys[a * D + b] = T3[a] * y1;
+                }
+            }
+            // FP64 folds, f = sub and c = sub factored out: sums over e (b)
+            // of one d (a), then over d (a)
+            R zu = 0, zv = 0, wu = 0, wv4 = 0, P2 = 0;
 #pragma unroll
             for (int rb = 0; rb < SH::RB; rb++) {
                 acc_t z = {0, 0, 0, 0}, w = {0, 0, 0, 0};
 #pragma unroll
                 for (int s = 0; s < SH::KS; s++) {
-                    const int a = s / D, b = s % D;
                     const R Az = Cl[LQ::at(4 * s + sub, 16 * rb + j)];
                     const R Aw = Cl[LQ::at(16 * rb + j, 4 * s + sub)];
-                    z = MA::op(Az, (T0[a] * T1[b]) * t2, z);
-                    w = MA::op(Aw, (T3[a] * T4[b]) * t5, w);
+                    z = MA::op(Az, xs[s], z);
+                    w = MA::op(Aw, ys[s], w);
                 }
                 if (MA::f64) {
                     // output row 16 rb + sub + 4 v: (d, e) or (a, b) = 4 rb + v, f or c = sub
@@ -481,14 +494,17 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_eval4m(int G, const int *__rest
                         const int de = 4 * rb + v;
                         if (de >= D * D) continue;
                         const int d = de / D, e = de % D;
-                        const R t34 = T3[d] * T4[e];
-                        S += z[v] * (t34 * t5);
-                        Gs[3] += z[v] * ((dT3[d] * T4[e]) * t5);
-                        Gs[4] += z[v] * ((T3[d] * dT4[e]) * t5);
-                        Gs[5] += z[v] * (t34 * dt5);
-                        Gs[0] += w[v] * ((dT0[d] * T1[e]) * t2);
-                        Gs[1] += w[v] * ((T0[d] * dT1[e]) * t2);
-                        Gs[2] += w[v] * ((T0[d] * T1[e]) * dt2);
+                        zu = e ? fma(T4[e], z[v], zu) : z[v];
+                        zv = e ? fma(dT4[e], z[v], zv) : 0;
+                        wu = e ? fma(T1[e], w[v], wu) : w[v];
+                        wv4 = e ? fma(dT1[e], w[v], wv4) : 0;
+                        if (e < D - 1) continue;
+                        S = fma(T3[d], zu, S);
+                        Gs[3] = fma(dT3[d], zu, Gs[3]);
+                        Gs[4] = fma(T3[d], zv, Gs[4]);
+                        P2 = fma(T0[d], wu, P2);
+                        Gs[0] = fma(dT0[d], wu, Gs[0]);
+                        Gs[1] = fma(T0[d], wv4, Gs[1]);
                     }
                 } else {
                     // output row 16 rb + 4 sub + v: (d, e) or (a, b) = 4 rb + sub, f or c = v
@@ -521,6 +537,15 @@ __global__ __launch_bounds__(64 * WPB, 2) void k_eval4m(int G, const int *__rest
                 }
                 // keep the operand loads of the next row block out of this one
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            if (MA::f64) {
+                Gs[5] = S * dt5;
+                S *= t5;
+                Gs[3] *= t5;
+                Gs[4] *= t5;
+                Gs[0] *= t2;
+                Gs[1] *= t2;
+                Gs[2] = P2 * dt2;
             }
         } else {
 #pragma unroll
