@@ -67,6 +67,7 @@ struct chx_enum_args {
 template <int NT>
 __global__ void k_enum(chx_enum_args x);
 __global__ void k_enum_big(chx_enum_args x);
+template <int OWN>
 __global__ void k_place(chx_enum_args x);
 __global__ void k_scan_block(const int *in, int *out, long n, int *bsum);
 __global__ void k_scan_add(int *out, long n, const int *bscan);

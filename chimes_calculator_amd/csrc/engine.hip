@@ -1347,7 +1347,8 @@ void run_pipeline(chx_engine *e, double *Fout, double *Ecfg, double *Vcfg)
         gb.status = e->status;
         e->scan(e->cnt34.p, e->off34.p, (long)(G3 + G4) * N, 0, gb);
         // every record to its list position
-        hipLaunchKernelGGL(k_place, dim3(nblk(N, 4)), dim3(256), 0, st, ea);
+        if (wide) hipLaunchKernelGGL((k_place<1>), dim3(nblk(N, 4)), dim3(256), 0, st, ea);
+        else hipLaunchKernelGGL((k_place<4>), dim3(nblk(N, 16)), dim3(256), 0, st, ea);
     }
     e->record(1);
     // evaluation with exact accumulation

@@ -324,10 +324,9 @@ __device__ __forceinline__ bool nbr_confirm(const chx_cfg &C, const chx_atom_n &
     return nbr_image(C, ni.u, an[(int)(k >> 24)].u, sh, zero, vn);
 }
 
-// Slab entry of image key k (both frames).
-__device__ __forceinline__ void nbr_write(const chx_cfg &C, const chx_atom_n &ni, const chx_atom_s *__restrict__ as,
-                                          const chx_atom_n *__restrict__ an, long long k, chx_entry_s *es,
-                                          chx_entry_n *en)
+// Slab entry of image key k of atom sa, at vn in the neighbour frame (both frames).
+__device__ __forceinline__ void nbr_store(const chx_cfg &C, const double *vn, const chx_atom_s &sa, long long k,
+                                          chx_entry_s *es, chx_entry_n *en)
 {
     const int a = (int)(k >> 24);
     const int spack = (int)(k & 0xffffff);
@@ -335,10 +334,9 @@ __device__ __forceinline__ void nbr_write(const chx_cfg &C, const chx_atom_n &ni
     unpack_shift(spack, sh);
     const bool zero = sh[0] == 0 && sh[1] == 0 && sh[2] == 0;
     chx_entry_n f;
-    nbr_image(C, ni.u, an[a].u, sh, zero, f.v);
+    f.v[0] = vn[0]; f.v[1] = vn[1]; f.v[2] = vn[2];
     f.shift = spack;
     f.pad = 0;
-    const chx_atom_s sa = as[a];
     chx_entry_s e;
     if (zero) {
         e.v[0] = sa.u[0]; e.v[1] = sa.u[1]; e.v[2] = sa.u[2];
@@ -355,11 +353,27 @@ __device__ __forceinline__ void nbr_write(const chx_cfg &C, const chx_atom_n &ni
     *en = f;
 }
 
+__device__ __forceinline__ void nbr_write(const chx_cfg &C, const chx_atom_n &ni, const chx_atom_s *__restrict__ as,
+                                          const chx_atom_n *__restrict__ an, long long k, chx_entry_s *es,
+                                          chx_entry_n *en)
+{
+    const int a = (int)(k >> 24);
+    int sh[3];
+    unpack_shift((int)(k & 0xffffff), sh);
+    double vn[3];
+    nbr_image(C, ni.u, an[a].u, sh, sh[0] == 0 && sh[1] == 0 && sh[2] == 0, vn);
+    nbr_store(C, vn, as[a], k, es, en);
+}
+
 // ---------------------------------------------------------------------------
 // Neighbour lists: for real atom i every image g = (a, n) with i <= a,
 // g != i and |r_g - r_i| < search in the neighbour frame
 // (serial_chimes_interface.cpp:682-731).  One wavefront per owner, four
 // owners per workgroup; lanes stride over the atoms of each searched cell.
+// Wavefronts are independent (wavefront-level fences only), and an owner with
+// at most 64 keys, the usual case, keeps its images in registers from the
+// exact test to the slab: bound by vector issue (fractional tests and frames),
+// 819 -> 760 us on the C/O batch of 4096 configurations.
 // Candidates that pass the cheap test are collected as (parent, shift) keys
 // in LDS, confirmed by the reference's arithmetic, ranked, and each owner's
 // images written sorted by key into its slab, so every list and every later
@@ -399,13 +413,13 @@ __global__ __launch_bounds__(256) void k_nbr(int natoms, const chx_cfg *__restri
     const chx_cfg &C = cfgs[own ? as[i].cfg : 0];
     int ci[3] = {0, 0, 0}, nc = 0, T = 0;
     // one candidate per lane: cheap test, keys of those that pass appended
-    auto take = [&](bool valid, int a, int spk) {
+    auto take = [&](bool valid, int a, int spk, const double *ua) {
         bool in = false;
         if (valid) {
             int sh[3];
             unpack_shift(spk, sh);
             const bool zero = sh[0] == 0 && sh[1] == 0 && sh[2] == 0;
-            if (!(a < i || (a == i && zero))) in = nbr_near(C, ni.u, an[a].u, sh);
+            if (!(a < i || (a == i && zero))) in = nbr_near(C, ni.u, ua, sh);
         }
         const unsigned long long b = __ballot(in);
         if (in) {
@@ -420,14 +434,28 @@ __global__ __launch_bounds__(256) void k_nbr(int natoms, const chx_cfg *__restri
         nc = (2 * C.reach[0] + 1) * (2 * C.reach[1] + 1) * (2 * C.reach[2] + 1);
         if (nc <= CHX_NBR_CELLS) T = nbr_cells(C, ci, ni.u, nc, lane, cell_start, cpre[wv], cadj[wv], cshf[wv], ccell[wv]);
     }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // each wavefront reads its own tables only
+    __builtin_amdgcn_wave_barrier();
     if (own) {
         if (nc <= CHX_NBR_CELLS) {
-            for (int t0 = 0; t0 < T; t0 += 64) {
-                const int t = t0 + lane;
-                int a = 0, spk = 0;
-                if (t < T) nbr_cand(t, T, nc, cpre[wv], cadj[wv], cshf[wv], ccell[wv], cell_atoms, a, spk);
-                take(t < T, a, spk);
+            // two candidates per lane a pass: their two dependent loads are
+            // in flight together
+            for (int t0 = 0; t0 < T; t0 += 128) {
+                int a[2], spk[2];
+#pragma unroll
+                for (int w = 0; w < 2; w++) {
+                    const int t = t0 + 64 * w + lane;
+                    a[w] = i;
+                    spk[w] = 0;
+                    if (t < T) nbr_cand(t, T, nc, cpre[wv], cadj[wv], cshf[wv], ccell[wv], cell_atoms, a[w], spk[w]);
+                }
+                double ua[2][3];
+#pragma unroll
+                for (int w = 0; w < 2; w++)
+#pragma unroll
+                    for (int k = 0; k < 3; k++) ua[w][k] = an[a[w]].u[k];
+                take(t0 + lane < T, a[0], spk[0], ua[0]);
+                if (t0 + 64 < T) take(t0 + 64 + lane < T, a[1], spk[1], ua[1]);
             }
         } else {
             for (int dz = -C.reach[2]; dz <= C.reach[2]; dz++)
@@ -438,13 +466,41 @@ __global__ __launch_bounds__(256) void k_nbr(int natoms, const chx_cfg *__restri
                         const int cs = cell_start[cell], ce = cell_start[cell + 1];
                         const int spk = pack_shift(sh);
                         for (int p0 = cs; p0 < ce; p0 += 64) {
-                            const int p = p0 + lane;
-                            take(p < ce, p < ce ? cell_atoms[p] : 0, spk);
+                            const int p = p0 + lane, a = p < ce ? cell_atoms[p] : i;
+                            take(p < ce, a, spk, an[a].u);
                         }
                     }
         }
     }
-    __syncthreads();
+    // at most one key per lane (the usual case): the reference's test, its
+    // image kept for the slab entry, and the entry's atom loaded while the
+    // keys are ranked
+    if (own && n1 <= 64) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const bool have = lane < n1;
+        const long long k = have ? keys[wv][lane] : ((long long)i << 24);
+        const int a = (int)(k >> 24);
+        int sh[3];
+        unpack_shift((int)(k & 0xffffff), sh);
+        double vn[3];
+        const bool in = nbr_image(C, ni.u, an[a].u, sh, sh[0] == 0 && sh[1] == 0 && sh[2] == 0, vn) && have;
+        const chx_atom_s sa = as[a];
+        if (have && !in) keys[wv][lane] = NBR_DROPPED;
+        const int n = __popcll(__ballot(in));
+        if (lane == 0) nbr_slab_note(i, n, nb_cap, nbr_cnt, nbr_off, status);
+        if (n > nb_cap) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        int rk = 0;
+        for (int q = 0; q < n1; q++) rk += keys[wv][q] < k;
+        const long at = (long)i * nb_cap + rk;
+        if (in) nbr_store(C, vn, sa, k, es + at, en + at);
+        return;
+    }
+    // more: rounds of 64 (wavefronts are independent here: their keys are their own)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     // the reference's test on the keys that passed; failures are marked
     int n = n1;
     if (own && n1 <= CHX_MAX_NB) {
@@ -460,7 +516,8 @@ __global__ __launch_bounds__(256) void k_nbr(int natoms, const chx_cfg *__restri
         }
     }
     if (own && lane == 0) nbr_slab_note(i, n, nb_cap, nbr_cnt, nbr_off, status);
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
     if (!own || n > CHX_MAX_NB || n > nb_cap) return;
     const long off = (long)i * nb_cap;
     for (int j = lane; j < n1; j += 64) {
@@ -895,44 +952,65 @@ __global__ __launch_bounds__(64) void k_enum_big(chx_enum_args x)
     }
 }
 
-// Records to list positions, one wavefront per owner: a record of group gg at
-// its slot goes to the group's base + the owner's offset within the group
-// (the scan of the counts) + the slot.  With few groups the owner's position
-// in each group is computed once, into LDS.
-constexpr int PLACE_GROUPS = 32;
-
+// Records to list positions, OWN owners per wavefront: a record of group
+// gg at its slot goes to the group's base + the owner's offset within the
+// group (the scan of the counts) + the slot.  With few groups the owners'
+// positions in each group are computed once, a lane each, into LDS.  The work
+// is a chain of short dependent loads (one owner a wavefront spent 90% of its
+// time waiting): in large batches four owners' loads are in flight together
+// (C/O batch of 4096 configurations, 39 M records, beside the 2-body kernel:
+// 345 -> 214 us); small batches keep an owner a wavefront, since they do not
+// fill the device otherwise (1536 water atoms: 6.6 us, 12 with four).
+template <int OWN>
 __global__ __launch_bounds__(256) void k_place(chx_enum_args x)
 {
-    __shared__ int pos[4][2][PLACE_GROUPS];
+    constexpr int PLACE_OWN = OWN, PLACE_GROUPS = 64 / OWN;
+    __shared__ int pos[4][PLACE_OWN][PLACE_GROUPS];
     if (block_stop(x.status, CHX_STOP)) return;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = (int)(blockIdx.x * 4 + wv);
+    const int i0 = (int)(blockIdx.x * 4 + wv) * PLACE_OWN;
     const int lane = threadIdx.x & 63;
     const long N = x.natoms;
-    const bool own = i < x.natoms;
-    const bool table = x.G3 <= PLACE_GROUPS && x.G4 <= PLACE_GROUPS;
-    if (own && table) {
-        if (lane < x.G3) pos[wv][0][lane] = x.gb3[lane] + (x.off3[lane * N + i] - x.off3[lane * N]);
-        else if (lane >= 32 && lane - 32 < x.G4)
-            pos[wv][1][lane - 32] = x.gb4[lane - 32] + (x.off4[(lane - 32) * N + i] - x.off4[(lane - 32) * N]);
+    const bool table = x.G3 + x.G4 <= PLACE_GROUPS;
+    if (table) {
+        const int o = lane / PLACE_GROUPS, t = lane % PLACE_GROUPS, i = i0 + o;
+        if (i < N && t < x.G3 + x.G4) {
+            const bool four = t >= x.G3;
+            const int g = four ? t - x.G3 : t;
+            const int *off = (four ? x.off4 : x.off3) + g * N;
+            pos[wv][o][t] = (four ? x.gb4 : x.gb3)[g] + (off[i] - off[0]);
+        }
     }
     __syncthreads();
-    if (!own) return;
-    const int n = uniform_load(x.nrec, i);
-    const int2 *rec = x.rec + (long)i * x.rcap;
-    for (int r = lane; r < n; r += 64) {
-        const int2 e = rec[r];
-        const int gg = (e.y >> 20) & 0x7ff;
-        const int slot = e.y & 0xfffff;
-        const bool four = e.y < 0;
-        int p;
-        if (table) p = pos[wv][four][gg];
-        else if (four) p = x.gb4[gg] + (x.off4[gg * N + i] - x.off4[gg * N]);
-        else p = x.gb3[gg] + (x.off3[gg * N + i] - x.off3[gg * N]);
-        (four ? x.list4 : x.list3)[p + slot] = make_int2(i, e.x);
+    int n[PLACE_OWN], most = 0;
+#pragma unroll
+    for (int o = 0; o < PLACE_OWN; o++) {
+        n[o] = i0 + o < N ? uniform_load(x.nrec, i0 + o) : 0;
+        most = max(most, n[o]);
+    }
+    for (int r = lane; r - lane < most; r += 64) {
+        int2 e[PLACE_OWN];
+#pragma unroll
+        for (int o = 0; o < PLACE_OWN; o++)
+            if (r < n[o]) e[o] = x.rec[(long)(i0 + o) * x.rcap + r];
+#pragma unroll
+        for (int o = 0; o < PLACE_OWN; o++) {
+            if (r >= n[o]) continue;
+            const int i = i0 + o;
+            const int gg = (e[o].y >> 20) & 0x7ff;
+            const int slot = e[o].y & 0xfffff;
+            const bool four = e[o].y < 0;
+            int p;
+            if (table) p = pos[wv][o][four ? x.G3 + gg : gg];
+            else if (four) p = x.gb4[gg] + (x.off4[gg * N + i] - x.off4[gg * N]);
+            else p = x.gb3[gg] + (x.off3[gg * N + i] - x.off3[gg * N]);
+            (four ? x.list4 : x.list3)[p + slot] = make_int2(i, e[o].x);
+        }
     }
 }
 
+template __global__ void k_place<1>(chx_enum_args);
+template __global__ void k_place<4>(chx_enum_args);
 template __global__ void k_enum<64>(chx_enum_args);
 template __global__ void k_enum<256>(chx_enum_args);
 
