@@ -25,6 +25,22 @@ __global__ void k_prep(int natoms, int ncfg, const int *cfg_atom_off, const chx_
                        const int *types, chx_atom_s *as, chx_atom_n *an, int *cell_count,
                        const int *cfg_item_off, int *in_cfg, int *item_cfg);
 __global__ void k_cell_fill(int natoms, const chx_atom_n *an, const int *cell_start, int *cursor, int *cell_atoms);
+// k_setup_small: clearing, k_prep, the cell scan and k_cell_fill of a batch of
+// at most CHX_SETUP_ATOMS atoms and fewer than CHX_SETUP_CELLS cells
+struct chx_setup_args {
+    int natoms, ncfg, ncell, nclear;
+    const chx_clear_range *clear;
+    const int *cfg_atom_off;
+    const chx_cfg *cfgs;
+    const double *pos;
+    const int *types;
+    chx_atom_s *as;
+    chx_atom_n *an;
+    const int *cfg_item_off;
+    int *in_cfg, *item_cfg;
+    int *cell_start, *cell_atoms;
+};
+__global__ void k_setup_small(chx_setup_args x);
 __global__ void k_nbr(int natoms, const chx_cfg *cfgs, const chx_atom_s *as, const chx_atom_n *an,
                       const int *cell_start, const int *cell_atoms, int *nbr_cnt, int *nbr_off, chx_entry_s *es,
                       chx_entry_n *en, int nb_cap, int *status);

@@ -67,6 +67,11 @@ struct chx_clear_range {
 // CHX_VAR_MFMAV names that FP32-mixed kernel too; where a matrix-core variant
 // does not apply the one-cluster-per-lane kernel stands in.
 enum { CHX_VAR_MFMA4 = 0, CHX_VAR_MFMA2 = 1, CHX_VAR_VECTOR = 2, CHX_VAR_MFMAV = 3, CHX_NVAR = 4 };
+// One-workgroup set-up (k_setup_small): atoms, cells (one less than this) and
+// ints to clear of the largest batch that takes it
+#define CHX_SETUP_ATOMS 1024
+#define CHX_SETUP_CELLS 4096
+#define CHX_SETUP_CLEAR 32768
 #define CHX_SCAN1_MAX 32768    // scans up to this length run in one workgroup
 
 // Per-configuration frame data (one per configuration in a batch).

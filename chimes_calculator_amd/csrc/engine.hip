@@ -1273,13 +1273,24 @@ void run_pipeline(chx_engine *e, double *Fout, double *Ecfg, double *Vcfg)
     };
     e->record(0);
     HIPCHK(hipMemcpyAsync(e->in_d.p, e->in_h.p, e->in_bytes, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_clear, dim3(1024), dim3(256), 0, st, e->clear, e->nclear);
-    hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, (int)N, ncfg, e->cfg_atom_off, e->cfgs,
-                       e->pos_in, e->types_in, e->as.p, e->an.p, e->cell_cnt.p, e->cfg_item_off, e->in_cfg.p,
-                       e->item_cfg.p);
-    e->scan(e->cell_cnt.p, e->cell_start.p, ncell);
-    hipLaunchKernelGGL(k_cell_fill, dim3(nblk(N, 256)), dim3(256), 0, st, (int)N, e->an.p, e->cell_start.p,
-                       e->cell_cur.p, e->cell_atoms.p);
+    // the whole set-up of a small batch is one launch
+    long to_clear = 0;
+    const chx_clear_range *cl = (const chx_clear_range *)(e->in_h.p + ((char *)e->clear - e->in_d.p));
+    for (int k = 0; k < e->nclear; k++) to_clear += cl[k].n;
+    if (N <= CHX_SETUP_ATOMS && ncell < CHX_SETUP_CELLS && to_clear <= CHX_SETUP_CLEAR) {
+        chx_setup_args sa{(int)N, ncfg, (int)ncell, e->nclear, e->clear, e->cfg_atom_off, e->cfgs, e->pos_in,
+                          e->types_in, e->as.p, e->an.p, e->cfg_item_off, e->in_cfg.p, e->item_cfg.p,
+                          e->cell_start.p, e->cell_atoms.p};
+        hipLaunchKernelGGL(k_setup_small, dim3(1), dim3(1024), 0, st, sa);
+    } else {
+        hipLaunchKernelGGL(k_clear, dim3(1024), dim3(256), 0, st, e->clear, e->nclear);
+        hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, (int)N, ncfg, e->cfg_atom_off, e->cfgs,
+                           e->pos_in, e->types_in, e->as.p, e->an.p, e->cell_cnt.p, e->cfg_item_off, e->in_cfg.p,
+                           e->item_cfg.p);
+        e->scan(e->cell_cnt.p, e->cell_start.p, ncell);
+        hipLaunchKernelGGL(k_cell_fill, dim3(nblk(N, 256)), dim3(256), 0, st, (int)N, e->an.p, e->cell_start.p,
+                           e->cell_cur.p, e->cell_atoms.p);
+    }
     // neighbour images, sorted per owner
     // small batches: one owner per workgroup (four wavefronts), else one per wavefront
     const bool wide = N <= CHX_ENUM_WIDE_MAX;

@@ -87,13 +87,12 @@ __global__ void k_fill_f64(double *p, long n)
 // ---------------------------------------------------------------------------
 // Atom preparation: one thread per replicated atom.
 // ---------------------------------------------------------------------------
-__global__ void k_prep(int natoms, int ncfg, const int *__restrict__ cfg_atom_off, const chx_cfg *__restrict__ cfgs,
-                       const double *__restrict__ pos, const int *__restrict__ types, chx_atom_s *as,
-                       chx_atom_n *an, int *cell_count, const int *__restrict__ cfg_item_off, int *in_cfg,
-                       int *item_cfg)
+// Replicated atom r: wrapped, in both frames, and its cell (returned).
+__device__ __forceinline__ int prep_atom(int r, int ncfg, const int *__restrict__ cfg_atom_off,
+                                         const chx_cfg *__restrict__ cfgs, const double *__restrict__ pos,
+                                         const int *__restrict__ types, chx_atom_s *as, chx_atom_n *an,
+                                         const int *__restrict__ cfg_item_off, int *in_cfg, int *item_cfg)
 {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= natoms) return;
     const int c = find_cfg(cfg_atom_off, ncfg, r);
     const chx_cfg &C = cfgs[c];
     const int l = r - C.atom_off;
@@ -137,7 +136,18 @@ __global__ void k_prep(int natoms, int ncfg, const int *__restrict__ cfg_atom_of
     n.cell = cell;
     n.orig = ain;
     an[r] = n;
-    atomicAdd(&cell_count[cell], 1);
+    return cell;
+}
+
+__global__ void k_prep(int natoms, int ncfg, const int *__restrict__ cfg_atom_off, const chx_cfg *__restrict__ cfgs,
+                       const double *__restrict__ pos, const int *__restrict__ types, chx_atom_s *as,
+                       chx_atom_n *an, int *cell_count, const int *__restrict__ cfg_item_off, int *in_cfg,
+                       int *item_cfg)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= natoms) return;
+    atomicAdd(&cell_count[prep_atom(r, ncfg, cfg_atom_off, cfgs, pos, types, as, an, cfg_item_off, in_cfg,
+                                    item_cfg)], 1);
 }
 
 __global__ void k_cell_fill(int natoms, const chx_atom_n *__restrict__ an, const int *__restrict__ cell_start,
@@ -148,6 +158,68 @@ __global__ void k_cell_fill(int natoms, const chx_atom_n *__restrict__ an, const
     const int c = an[r].cell;
     const int p = atomicAdd(&cursor[c], 1);
     cell_atoms[cell_start[c] + p] = r;
+}
+
+// Clearing, preparation, the cell scan and the cell lists of a small batch in
+// one workgroup, cell counts in LDS: for a few hundred atoms each of the four
+// launches it replaces is shorter than the launch itself (64 atoms: 2.8 + 2.8
+// + 5.8 + 2.2 us and three gaps against 5.3 us; a calculator call of 64 atoms
+// 155 -> 142 us, a plan of 729 carbon atoms 144 -> 132 us).  Up to
+// CHX_SETUP_ATOMS atoms, one a thread, and as many cells and words to clear as
+// one workgroup passes over in a few microseconds.
+__global__ __launch_bounds__(1024) void k_setup_small(chx_setup_args x)
+{
+    __shared__ int cnt[CHX_SETUP_CELLS];
+    __shared__ int wsum[16];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    for (int k = 0; k < x.nclear; k++) {
+        int *p = x.clear[k].p;
+        const int n = (int)x.clear[k].n;
+        for (int i = tid; i < n; i += 1024) p[i] = 0;
+    }
+    for (int c = tid; c < CHX_SETUP_CELLS; c += 1024) cnt[c] = 0;
+    __syncthreads();
+    int cell[CHX_SETUP_ATOMS / 1024];
+#pragma unroll
+    for (int u = 0; u < CHX_SETUP_ATOMS / 1024; u++) {
+        const int r = tid + 1024 * u;
+        cell[u] = -1;
+        if (r < x.natoms) {
+            cell[u] = prep_atom(r, x.ncfg, x.cfg_atom_off, x.cfgs, x.pos, x.types, x.as, x.an, x.cfg_item_off,
+                                x.in_cfg, x.item_cfg);
+            atomicAdd(&cnt[cell[u]], 1);
+        }
+    }
+    __syncthreads();
+    // exclusive scan of the counts, a contiguous segment per thread
+    constexpr int PER = CHX_SETUP_CELLS / 1024;
+    int v[PER], t = 0;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        v[q] = cnt[tid * PER + q];
+        t += v[q];
+    }
+    int s = t;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(s, d, 64);
+        if (lane >= d) s += y;
+    }
+    if (lane == 63) wsum[w] = s;
+    __syncthreads();
+    int run = s - t;
+    for (int k = 0; k < w; k++) run += wsum[k];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int c = tid * PER + q;
+        if (c <= x.ncell) x.cell_start[c] = run;
+        cnt[c] = run;
+        run += v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < CHX_SETUP_ATOMS / 1024; u++)
+        if (cell[u] >= 0) x.cell_atoms[atomicAdd(&cnt[cell[u]], 1)] = tid + 1024 * u;
 }
 
 // Image of atom a under lattice shift sh in the neighbour frame, and whether
