@@ -338,16 +338,12 @@ int chimes_gpu_compute_clusters(chimes_gpu_model *m, int nb, int n, const double
                                 const int *types, double *energy, double *force, double *stress)
 {
     if (nb < 2 || nb > 4) return fail("cluster size must be 2, 3 or 4");
-    const int P = nb * (nb - 1) / 2;
     const int nt = m->dm->P.natmtyps;
     for (long k = 0; k < (long)n * nb; k++)
         if (types[k] < 0 || types[k] >= nt) return fail("atom type index out of range");
-    std::vector<double> last((size_t)n * P, 0.0);
-    std::vector<int> flags(n);
     chx::EngineHandle *eh = m->dm->eh;
     std::lock_guard<std::mutex> lk(eh->mu);
-    if (chx_eval_clusters(eh->eng, m->dm->m, nb, n, dist, dr, types, energy, force, stress, last.data(),
-                          flags.data()))
+    if (chx_eval_clusters(eh->eng, m->dm->m, nb, n, dist, dr, types, energy, force, stress, nullptr, nullptr))
         return fail(chx_last_error(eh->eng));
     return 0;
 }

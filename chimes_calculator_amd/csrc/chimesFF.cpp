@@ -140,13 +140,9 @@ void chimesFF::compute_clusters(int nb, int n, const double *dx, const double *d
 {
     require_model("compute_clusters");
     if (n <= 0) return;
-    const int P = nb * (nb - 1) / 2;
-    std::vector<double> last((size_t)n * P, 0.0);
-    std::vector<int> flags(n);
     chx::DeviceModel &dm = *impl_->dm;
     std::lock_guard<std::mutex> lk(dm.eh->mu);
-    if (chx_eval_clusters(dm.eh->eng, dm.m, nb, n, dx, dr, typ_idxs, energy, force, stress, last.data(),
-                          flags.data()))
+    if (chx_eval_clusters(dm.eh->eng, dm.m, nb, n, dx, dr, typ_idxs, energy, force, stress, nullptr, nullptr))
         fatal(chx_last_error(dm.eh->eng));
 }
 

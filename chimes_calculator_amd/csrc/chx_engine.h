@@ -92,7 +92,8 @@ void chx_free(void *p);
 // Explicit clusters (the per-cluster API): nb = 2, 3 or 4 bodies, n clusters.
 // dist[n*P], dr[n*P*3], types[n*nb]; outputs energy[n], force[n*nb*3],
 // stress[n*6] (packed xx xy xz yy yz zz), last[n*P] (last-term scalars,
-// 2-body: penalty scalar), flags[n].
+// 2-body: penalty scalar), flags[n]; last and flags may be null together: not
+// wanted.
 int chx_eval_clusters(chx_engine *e, chx_model *m, int nb, int n, const double *dist, const double *dr,
                       const int *types, double *energy, double *force, double *stress, double *last,
                       int *flags);

@@ -46,6 +46,7 @@ void launch_evalv(int nb, int D, int prec, const chx_list_args &la, hipStream_t 
 void launch_eval_body(int nb, int D, int prec, int variant, const chx_list_args &la, hipStream_t st);
 // Whether variant names a kernel of its own (CHX_VAR_MFMAV is CHX_VAR_VECTOR's).
 bool variant_applies(int variant);
+// last and flags null: not wanted (neither computed nor written)
 void launch_clusters(int nb, int D, int n, hipStream_t st, const double *dist, const double *drv, const int *types,
                      const chx_model_dev &M, double *E, double *F, double *S, double *last, int *flags);
 

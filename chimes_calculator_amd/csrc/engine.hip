@@ -1968,17 +1968,12 @@ int chx_eval_clusters_static(chx_engine *e, chx_model *m, int nb, int n, const d
         double *oE = (double *)take(sizeof(double) * n);
         double *oF = (double *)take(sizeof(double) * n * nb * 3);
         double *oS = (double *)take(sizeof(double) * n * 6);
-        double *oL = (double *)take(sizeof(double) * n * P);
-        int *oflags = (int *)take(sizeof(int) * n);
         if (off > CHX_SCRATCH_BYTES) throw EngineError("scratch layout exceeds the scratch array");
         HIPCHK(hipMemcpyAsync(d_dist, dist, sizeof(double) * n * P, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_dr, dr, sizeof(double) * n * P * 3, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_types, types, sizeof(int) * n * nb, hipMemcpyHostToDevice, st));
-        // the last-term scalars keep their value for a cluster that is not
-        // evaluated: they start at zero, as chimes_gpu_compute_clusters's do
-        hipLaunchKernelGGL(k_fill_f64, dim3(nblk((long)n * P, 256)), dim3(256), 0, st, oL, (long)n * P);
         launch_clusters(nb, nb == 3 ? m->d.D3 : (nb == 4 ? m->d.D4 : 2), n, st, d_dist, d_dr, d_types, m->dev, oE,
-                        oF, oS, oL, oflags);
+                        oF, oS, nullptr, nullptr);
         HIPCHK(hipMemcpyAsync(energy, oE, sizeof(double) * n, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(force, oF, sizeof(double) * n * nb * 3, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(stress, oS, sizeof(double) * n * 6, hipMemcpyDeviceToHost, st));
@@ -2003,22 +1998,24 @@ int chx_eval_clusters(chx_engine *e, chx_model *m, int nb, int n, const double *
         const int P = nb * (nb - 1) / 2;
         hipStream_t st = e->st;
         e->cl_in.ensure((size_t)n * P * 4);
-        e->cl_out.ensure((size_t)n * (1 + 3 * nb + 6 + P));
+        e->cl_out.ensure((size_t)n * (1 + 3 * nb + 6 + (last ? P : 0)));
         e->cl_types.ensure((size_t)n * nb);
-        e->cl_flags.ensure(n);
+        if (last) e->cl_flags.ensure(n);
         double *d_dist = e->cl_in.p, *d_dr = e->cl_in.p + (size_t)n * P;
         double *oE = e->cl_out.p, *oF = oE + n, *oS = oF + (size_t)n * nb * 3, *oL = oS + (size_t)n * 6;
         HIPCHK(hipMemcpyAsync(d_dist, dist, sizeof(double) * n * P, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(d_dr, dr, sizeof(double) * n * P * 3, hipMemcpyHostToDevice, st));
         HIPCHK(hipMemcpyAsync(e->cl_types.p, types, sizeof(int) * n * nb, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(oL, last, sizeof(double) * n * P, hipMemcpyHostToDevice, st));
+        if (last) HIPCHK(hipMemcpyAsync(oL, last, sizeof(double) * n * P, hipMemcpyHostToDevice, st));
         launch_clusters(nb, nb == 3 ? m->d.D3 : (nb == 4 ? m->d.D4 : 2), n, st, d_dist, d_dr, e->cl_types.p, m->dev,
-                        oE, oF, oS, oL, e->cl_flags.p);
+                        oE, oF, oS, last ? oL : nullptr, last ? e->cl_flags.p : nullptr);
         HIPCHK(hipMemcpyAsync(energy, oE, sizeof(double) * n, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(force, oF, sizeof(double) * n * nb * 3, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(stress, oS, sizeof(double) * n * 6, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(last, oL, sizeof(double) * n * P, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipMemcpyAsync(flags, e->cl_flags.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+        if (last) {
+            HIPCHK(hipMemcpyAsync(last, oL, sizeof(double) * n * P, hipMemcpyDeviceToHost, st));
+            HIPCHK(hipMemcpyAsync(flags, e->cl_flags.p, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+        }
         HIPCHK(hipStreamSynchronize(st));
         HIPCHK(hipGetLastError());
         return 0;

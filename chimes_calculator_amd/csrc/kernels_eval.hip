@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(256) void k_fin(int ncfg, int nitems, const int *__
 // chimesFF.cpp:2171-2173, 2864-2869) and, for 2 bodies, the penalty scalar
 // (chimesFF.cpp:1745-1774).
 // ---------------------------------------------------------------------------
-template <int NB, int D>
+template <int NB, int D, bool LAST>
 __global__ __launch_bounds__(128) void k_clusters(int n, const double *__restrict__ dist, const double *__restrict__ drv,
                            const int *__restrict__ types, chx_model_dev M, double *E, double *F, double *Sout,
                            double *last, int *flags_out)
@@ -1075,12 +1075,12 @@ __global__ __launch_bounds__(128) void k_clusters(int n, const double *__restric
     double Ec, fo[NB][3], So[6];
     int flags = 0;
     bool evaluated;
-    explicit_cluster<NB, D>(M, ty, rq, dr, Ec, fo, So, flags, evaluated, last + (long)c * P);
+    explicit_cluster<NB, D>(M, ty, rq, dr, Ec, fo, So, flags, evaluated, LAST ? last + (long)c * P : nullptr);
     E[c] = Ec;
     for (int a = 0; a < NB; a++)
         for (int k = 0; k < 3; k++) F[((long)c * NB + a) * 3 + k] = fo[a][k];
     for (int k = 0; k < 6; k++) Sout[(long)c * 6 + k] = So[k];
-    flags_out[c] = flags | (evaluated ? 8 : 0);
+    if (LAST) flags_out[c] = flags | (evaluated ? 8 : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1176,24 +1176,27 @@ void launch_clusters(int nb, int D, int n, hipStream_t st, const double *dist, c
 {
     if (n <= 0) return;
     const dim3 grid((unsigned)((n + 127) / 128)), block(128);
+#define L(NB_, d)                                                                                             \
+    if (D == d) {                                                                                             \
+        if (last)                                                                                             \
+            hipLaunchKernelGGL((k_clusters<NB_, d, true>), grid, block, 0, st, n, dist, drv, types, M, E, F, S, \
+                               last, flags);                                                                  \
+        else                                                                                                  \
+            hipLaunchKernelGGL((k_clusters<NB_, d, false>), grid, block, 0, st, n, dist, drv, types, M, E, F, S, \
+                               last, flags);                                                                  \
+        return;                                                                                               \
+    }
     if (nb == 2) {
-        hipLaunchKernelGGL((k_clusters<2, 2>), grid, block, 0, st, n, dist, drv, types, M, E, F, S, last, flags);
-        return;
+        D = 2;
+        L(2, 2)
     }
-#define X(d)                                                                                                 \
-    if (D == d) {                                                                                            \
-        hipLaunchKernelGGL((k_clusters<3, d>), grid, block, 0, st, n, dist, drv, types, M, E, F, S, last, flags); \
-        return;                                                                                              \
-    }
+#define X(d) L(3, d)
     if (nb == 3) { CHX_D3_CASES(X) }
 #undef X
-#define X(d)                                                                                                 \
-    if (D == d) {                                                                                            \
-        hipLaunchKernelGGL((k_clusters<4, d>), grid, block, 0, st, n, dist, drv, types, M, E, F, S, last, flags); \
-        return;                                                                                              \
-    }
+#define X(d) L(4, d)
     if (nb == 4) { CHX_D4_CASES(X) }
 #undef X
+#undef L
 }
 
 }  // namespace chx
