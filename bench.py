@@ -599,7 +599,7 @@ def bench_c2(args):
     flops = nclus * term_flops(terms, d3 if body == 3 else d4, 3 if body == 3 else 6)
     ms = kt["3body"] if body == 3 else kt["4body"]
     peak = PEAK_FP32 if f32 else PEAK_FP64
-    prof = "%s_co4096_%s_counters.md" % ("k_evalv3" if body == 3 else "k_evalv4", "mixed" if f32 else "fp64")
+    prof = "k_lane_co4096_mixed_counters.md" if f32 else "k_evalv3_co4096_fp64_counters.md"
     figs = profile_figures(prof, kname.replace(" ", ""))
     traffic = (figs["fetch_bytes"] + figs["write_bytes"]) if "fetch_bytes" in figs else None
     # bound from the committed counters: HBM when the measured traffic would
