@@ -259,8 +259,8 @@ __device__ __forceinline__ void lane_contract4(const float *__restrict__ img, co
 // consecutive tiles share is flushed once.  C/O batch of 4096 configurations
 // (26.3 M triplets, 13.2 M quadruplets): 3-body D = 7 1.60 ms on the vector
 // ALU, 1.63 ms here with one tile, 1.43 with four, 1.41 with eight; 4-body
-// D = 3 1.33 ms on the vector ALU, 1.27 with four, 1.29 with eight (1.16 since
-// the recurrences and splits were shortened).  Carbon,
+// D = 3 1.33 ms on the vector ALU, 1.27 with four, 1.29 with eight (1.17 since
+// the exact splits were shortened).  Carbon,
 // 32768 atoms: 3-body D = 10 156 -> 129 us, 4-body D = 4 202 -> 167 us.
 //
 // The file is compiled without the hoisting of constants out of that loop
