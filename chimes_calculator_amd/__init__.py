@@ -181,6 +181,7 @@ class GpuModel:
     def types_to_index(self, types):
         # one library call per element name, not per atom: a batch of 64
         # configurations spent 2 of its 2.6 ms in those calls
+        types = types if hasattr(types, "__len__") else list(types)
         lut = {t: self.type_index(t) for t in set(types)}
         idx = np.fromiter(map(lut.__getitem__, types), np.int32, len(types))
         if any(k < 0 for k in lut.values()):

@@ -58,3 +58,24 @@ def test_caller_programs_build(tmp_path, name):
     from conftest import build_driver
     exe = build_driver(name, tmp_path)
     assert os.access(exe, os.X_OK)
+
+
+@pytest.mark.parametrize("form", [list, tuple, iter, lambda t: (x for x in t), lambda t: __import__("numpy").array(t)])
+def test_types_of_any_iterable(form):
+    """Element names of a configuration come as any iterable, one-shot ones
+    included; an unknown name is an error that names it."""
+    import chimes_calculator_amd as cc
+
+    class Model(cc.GpuModel):
+        h = None
+
+        def __init__(self):
+            pass
+
+        def type_index(self, name):
+            return {"C": 0, "O": 1}.get(name, -1)
+
+    assert Model().types_to_index(form(["O", "C", "C", "O"])).tolist() == [1, 0, 0, 1]
+    assert Model().types_to_index(form([])).tolist() == []
+    with pytest.raises(cc.ChimesError, match="Xx"):
+        Model().types_to_index(form(["C", "Xx"]))
