@@ -136,10 +136,10 @@ __device__ __forceinline__ double lmp_wave_sum(double x)
 // count, in row order, and evaluates 64 at a time, where lanes striding over
 // the row each did a few of many passes.  The owner's force and tallies are
 // summed over its lanes in double in that fixed order and added exactly once;
-// the partners' go through the workgroup's table.  4096 carbon atoms, order
-// 20, 184-entry rows: 40 us with energy and virial, where sixteen striding
-// lanes per owner and atomics to memory took 73 us (1728 atoms with per-atom
-// tallies: 30 us, before 102 us).  TAB: the pair's energy and force scalar
+// the partners' go through the workgroup's table.  2744 carbon atoms, order
+// 20, energy and virial: 22 us with rows of 161 entries and 13 with rows of 27,
+// where sixteen striding lanes per owner and atomics to memory took 54 and 15.
+// (With 112 bytes of scratch per lane, 23 and 15.)  TAB: the pair's energy and force scalar
 // come from its table (compute_2B_tab, chimesFF.cpp:1782-1856: cutoff test,
 // table lookups, no penalty term).
 // ---------------------------------------------------------------------------
@@ -235,10 +235,10 @@ __global__ __launch_bounds__(256) void k_lmp_pair(chx_lmp_args A, chx_model_dev 
                 for (int k = 0; k < 6; k++) fx_atomic(A.Vacc + 2L * (6L * i + k), v[k] / 2, bad);
         }
         // lane 0 the pairs' energy and virial, lane 1 the 1-body energy
-        const double z[6] = {0, 0, 0, 0, 0, 0}, ev = lane ? e1 : tot[3];
+        const double ev = lane ? e1 : tot[3];
         double gv[6];
 #pragma unroll
-        for (int k = 0; k < 6; k++) gv[k] = lane ? z[k] : v[k];
+        for (int k = 0; k < 6; k++) gv[k] = lane ? 0.0 : v[k];  // an array of zeros here would put both in scratch
         lmp_global_add(A, lane < 2, ev, gv, blockIdx.x & (CHX_LMP_GSLOTS - 1), bad);
     }
     __syncthreads();
