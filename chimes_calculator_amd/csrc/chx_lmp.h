@@ -43,9 +43,10 @@ struct chx_lmp_args {
 // T: the tables of a -DTABULATION build (null or empty: the polynomials)
 void launch_lmp_pair(const chx_lmp_args &A, const chx_model_dev &M, const chx_tabs_dev *T, hipStream_t st);
 // mode 0: per-owner counts into cnt3 / cnt4; mode 1: lists written at off3 /
-// off4; max_row: the longest neighbour row
-void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, double pad3, double pad4, int has4, int *cnt3, int *cnt4,
-                      const long long *off3, const long long *off4, int *trips, int *quads, hipStream_t st);
+// off4; max_row: the longest neighbour row, entries: all rows' entries
+void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, long entries, double pad3, double pad4, int has4,
+                      int *cnt3, int *cnt4, const long long *off3, const long long *off4, int *trips, int *quads,
+                      hipStream_t st);
 // rc: the largest cutoff of the body order; near[n] and *count (zeroed):
 // scratch for the clusters within it
 void launch_lmp_clusters(int nb, int D, long n, const int *list, double rc, int *near, int *count,

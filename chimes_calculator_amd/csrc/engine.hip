@@ -2184,7 +2184,9 @@ void lmp_build(chx_lmp *p, double skin)
     p->cnt.ensure((size_t)2 * inum + CHX_LMP_ST_WORDS);
     int max_row = 0;
     for (int ii = 0; ii < inum; ii++) max_row = std::max(max_row, p->off_h[ii + 1] - p->off_h[ii]);
-    launch_lmp_lists(0, A, max_row, pad3, pad4, has4, p->cnt.p, p->cnt.p + inum, nullptr, nullptr, nullptr, nullptr, st);
+    const long entries = p->off_h[inum];
+    launch_lmp_lists(0, A, max_row, entries, pad3, pad4, has4, p->cnt.p, p->cnt.p + inum, nullptr, nullptr, nullptr,
+                     nullptr, st);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(p->cnt.p + 2 * inum, p->status.p, sizeof(int) * CHX_LMP_ST_WORDS, hipMemcpyDeviceToDevice,
                           st));
@@ -2211,8 +2213,8 @@ void lmp_build(chx_lmp *p, double skin)
     p->trips.ensure(std::max<size_t>((size_t)t3 * 3, 3));
     p->quads.ensure(std::max<size_t>((size_t)t4 * 4, 4));
     HIPCHK(hipMemcpyAsync(p->off.p, p->scan_h.data(), sizeof(long long) * 2 * inum, hipMemcpyHostToDevice, st));
-    launch_lmp_lists(1, A, max_row, pad3, pad4, has4, nullptr, nullptr, p->off.p, p->off.p + inum, p->trips.p, p->quads.p,
-                     st);
+    launch_lmp_lists(1, A, max_row, entries, pad3, pad4, has4, nullptr, nullptr, p->off.p, p->off.p + inum, p->trips.p,
+                     p->quads.p, st);
     HIPCHK(hipGetLastError());
     p->have_lists = true;
 }

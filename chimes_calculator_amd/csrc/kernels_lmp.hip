@@ -40,6 +40,8 @@ __device__ __forceinline__ void lmp_order(const double (&s)[6], double (&v)[6])
 // dynamic LDS.  An atom that finds no slot within LMP_PROBES goes straight to
 // memory.
 constexpr int LMP_PROBES = 32;
+constexpr int LMP_SHORT_ROW = 64;   // candidates of an owner the one-wavefront list form holds
+constexpr int LMP_BRIEF_MEAN = 80;  // mean row length up to which it goes first
 
 struct lmp_table {
     int cap, nw;               // slots (a power of two), words per slot: 6 or 20
@@ -261,9 +263,10 @@ __global__ __launch_bounds__(256) void k_lmp_pair(chx_lmp_args A, chx_model_dev 
 // written in the reference's loop order.
 //
 // MODE 0 counts per owner, MODE 1 writes at the scanned offsets.  CAP bounds
-// |J|: the small form (29 KB of LDS, five owners a CU) takes owners with at
+// |J|: the small form (32 KB of LDS, four owners a CU) takes owners with at
 // most CAP, the large one those above `lo`; it is launched only when a row is
-// long enough.  1728 atoms at 3.2 g/cc, pads 5.5 / 4.625 A: 67 us
+// long enough, and neither where the one-wavefront form below took every
+// owner.  1728 atoms at 3.2 g/cc, pads 5.5 / 4.625 A: 67 us
 // to count and 147 us to write, where one wavefront per owner testing every l
 // of every pair took 1286 and 1465 us; the writes are now 53 MB in runs of a
 // few entries per lane.
@@ -429,6 +432,118 @@ __global__ __launch_bounds__(256) void k_lmp_lists(chx_lmp_args A, int lo, doubl
             }
             p4 += __shfl(s4, 63, 64);
         }
+    }
+}
+
+// The same lists for owners with at most 64 candidates, one wavefront per
+// owner.  The row-wise form above gives a wavefront one row of at most m pairs
+// at a time, a few lanes' worth where rows are short; here the m^2 pairs of
+// (a, b) are taken 64 at a time in list order, the 3-body entries come straight
+// from the ballots, and only the 4-body bits are kept as rows.  Bound by its
+// dependent loads and LDS reads.  Both passes, 8000 carbon atoms at 0.5 g/cc:
+// 25 us against 98 us with the row-wise form (20 and 94 without 4-body terms).
+template <int MODE>
+__global__ __launch_bounds__(64) void k_lmp_lists_short(chx_lmp_args A, double pad3, double pad4, int has4,
+                                                        int *cnt3, int *cnt4, const long long *off3,
+                                                        const long long *off4, int *trips, int *quads)
+{
+    constexpr int CAP = LMP_SHORT_ROW;
+    static_assert(CAP == 64, "a 4-body row is one word");
+    __shared__ double cx[CAP][3], cd[CAP];
+    __shared__ int cj[CAP], ctag[CAP];
+    __shared__ unsigned long long r4[CAP];
+    const int ii = blockIdx.x, lane = threadIdx.x;
+    const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const int i = A.ilist[ii], itag = A.tag[i];
+    const double xi[3] = {A.x[3L * i], A.x[3L * i + 1], A.x[3L * i + 2]};
+    const int beg = A.nbr_off[ii], n = A.nbr_off[ii + 1] - beg;
+    r4[lane] = 0ull;
+    int m = 0;
+    for (int b0 = 0; b0 < n; b0 += 64) {
+        bool v = false;
+        int j = 0, tj = 0;
+        double xj[3] = {0, 0, 0}, d = 0.0;
+        if (b0 + lane < n) {
+            j = A.nbr[beg + b0 + lane];
+            tj = A.tag[j];
+            if (j != i && tj >= itag) {
+                xj[0] = A.x[3L * j]; xj[1] = A.x[3L * j + 1]; xj[2] = A.x[3L * j + 2];
+                double dr[3];
+                d = lmp_dist(xi, xj, dr);
+                v = !(d >= pad3 && d >= pad4);
+            }
+        }
+        const unsigned long long bal = __ballot(v);
+        const int r = m + __popcll(bal & below);
+        if (v && r < CAP) {
+            cj[r] = j;
+            ctag[r] = tj;
+            cx[r][0] = xj[0]; cx[r][1] = xj[1]; cx[r][2] = xj[2];
+            cd[r] = d;
+        }
+        m += __popcll(bal);
+    }
+    if (m > CAP) return;  // the row-wise form takes it
+    __syncthreads();
+    const int total = m * m;
+    const float rm = 1.0f / (float)m;  // (p + 1/2) rm is at least 1/128 from a whole number, p < 4096: its floor is p / m
+    long long o3 = MODE ? off3[ii] : 0, o4 = MODE ? off4[ii] : 0;
+    int c3 = 0;
+    for (int p0 = 0; p0 < total; p0 += 64) {
+        const int p = p0 + lane;
+        bool v3 = false, v4 = false;
+        int a = 0, b = 0;
+        if (p < total) {
+            a = (int)(((float)p + 0.5f) * rm);
+            b = p - a * m;
+            if (cj[a] != cj[b] && ctag[b] >= ctag[a]) {
+                double dr[3];
+                const double dab = lmp_dist(cx[a], cx[b], dr), da = cd[a], db = cd[b];
+                v3 = da < pad3 && db < pad3 && dab < pad3;
+                v4 = has4 && da < pad4 && db < pad4 && dab < pad4;
+            }
+        }
+        const unsigned long long b3 = __ballot(v3);
+        if (MODE && v3) {
+            int *t = trips + 3 * (o3 + c3 + __popcll(b3 & below));
+            t[0] = i; t[1] = cj[a]; t[2] = cj[b];
+        }
+        c3 += __popcll(b3);
+        if (v4) atomicOr(&r4[a], 1ull << b);
+    }
+    __syncthreads();
+    int c4 = 0;
+    if (has4) {
+        for (int p0 = 0; p0 < total; p0 += 64) {
+            const int p = p0 + lane;
+            unsigned long long l = 0ull;
+            int a = 0, b = 0;
+            if (p < total) {
+                a = (int)(((float)p + 0.5f) * rm);
+                b = p - a * m;
+                if ((r4[a] >> b) & 1) l = r4[a] & r4[b];
+            }
+            if (__ballot(l != 0ull) == 0) continue;
+            const int c = __popcll(l);
+            int s4 = c;
+            for (int s = 1; s < 64; s <<= 1) {
+                const int u4 = __shfl_up(s4, s, 64);
+                if (lane >= s) s4 += u4;
+            }
+            if (MODE && c) {
+                int4 *u = reinterpret_cast<int4 *>(quads) + (o4 + c4 + s4 - c);
+                const int ja = cj[a], jb = cj[b];
+                while (l) {
+                    *u++ = make_int4(i, ja, jb, cj[__ffsll((long long)l) - 1]);
+                    l &= l - 1;
+                }
+            }
+            c4 += __shfl(s4, 63, 64);
+        }
+    }
+    if (MODE == 0 && lane == 0) {
+        cnt3[ii] = c3;
+        cnt4[ii] = c4;
     }
 }
 
@@ -779,22 +894,36 @@ void launch_lmp_pair(const chx_lmp_args &A, const chx_model_dev &M, const chx_ta
     else hipLaunchKernelGGL(k_lmp_pair<false>, grid, block, lds, st, A, M, chx_tabs_dev{});
 }
 
-void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, double pad3, double pad4, int has4, int *cnt3,
-                      int *cnt4, const long long *off3, const long long *off4, int *trips, int *quads, hipStream_t st)
+void launch_lmp_lists(int mode, const chx_lmp_args &A, int max_row, long entries, double pad3, double pad4, int has4,
+                      int *cnt3, int *cnt4, const long long *off3, const long long *off4, int *trips, int *quads,
+                      hipStream_t st)
 {
     if (A.inum <= 0) return;
     constexpr int SMALL = CHX_LMP_CAND / 2;
     const dim3 grid((unsigned)A.inum), block(256);
+    // Rows of up to 80 entries on average hold 64 candidates or fewer for
+    // nearly every owner.  2744 atoms, both passes, row-wise form alone against
+    // one wavefront per owner first: rows of 27 entries 43 against 18 us, 53:
+    // 60 and 36, 77: 71 and 64, 85: 102 and 128 (without 4-body terms 41 and
+    // 14, 53 and 21, 60 and 41, 87 and 76, but rows of 110 134 and 154).
+    const bool brief = entries <= (long)LMP_BRIEF_MEAN * A.inum;
+    const int lo = brief ? LMP_SHORT_ROW : -1;
+#define SHORT(MODE_)                                                                                           \
+    hipLaunchKernelGGL(k_lmp_lists_short<MODE_>, grid, dim3(64), 0, st, A, pad3, pad4, has4, cnt3, cnt4, off3, off4, \
+                       trips, quads)
 #define L(CAP_, MODE_, LO_)                                                                                    \
     hipLaunchKernelGGL((k_lmp_lists<CAP_, MODE_>), grid, block, 0, st, A, LO_, pad3, pad4, has4, cnt3, cnt4, off3, \
                        off4, trips, quads)
     if (mode == 0) {
-        L(SMALL, 0, -1);
+        if (brief) SHORT(0);
+        if (max_row > lo) L(SMALL, 0, lo);
         if (max_row > SMALL) L(CHX_LMP_CAND, 0, SMALL);
     } else {
-        L(SMALL, 1, -1);
+        if (brief) SHORT(1);
+        if (max_row > lo) L(SMALL, 1, lo);
         if (max_row > SMALL) L(CHX_LMP_CAND, 1, SMALL);
     }
+#undef SHORT
 #undef L
 }
 

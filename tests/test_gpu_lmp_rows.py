@@ -39,6 +39,49 @@ def test_rows(tmp_path, natoms, rc4):
     model.close()
 
 
+@pytest.mark.parametrize("ball,orders", [(0, (4, 3, 3)), (64, (4, 3, 3)), (65, (4, 3, 3)), (66, (4, 3, 3)),
+                                         (66, (4, 3, 0)), (258, (4, 3, 3)), (513, (4, 3, 0))])
+def test_short_rows(tmp_path, ball, orders):
+    """Rows of a few entries on average, which the one-wavefront list form
+    takes, beside a ball whose centre, of the lowest tag, has ball - 1
+    candidates: the most that form holds, and the owners it leaves to both
+    working sets of the row-wise form."""
+    from chimes_calculator_amd import GpuModel, LmpPair
+    rc4 = 2.0 if ball < 100 else 0.8
+    m = W.Model("short", ["C"], orders, (5.0, 4.0, rc4 if orders[2] else 0.0), {frozenset(("C",)): 0.05}, seed=ball)
+    pf = m.write(str(tmp_path / "short.txt"))
+    rng = np.random.default_rng(ball)
+    grid = (np.stack(np.meshgrid(*[np.arange(6)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5) * 8.0
+    grid = grid[np.linalg.norm(grid - 28.0, axis=1) > 7.0]
+    x = np.concatenate([g + rng.uniform(-0.6, 0.6, (k, 3)) for g, k in zip(grid, rng.integers(1, 6, len(grid)))])
+    tag = rng.permutation(len(x)).astype(np.int32) + 1 + ball
+    if ball:
+        v = rng.normal(size=(ball, 3))
+        r = 2.2 * rng.random((ball, 1)) ** (1.0 / 3.0)
+        r[0] = 0.0
+        x = np.concatenate([28.0 + v / np.linalg.norm(v, axis=1)[:, None] * r, x])
+        tag = np.concatenate([1 + np.arange(ball, dtype=np.int32), tag])
+    O = LmpOracle(pf)
+    S = LmpSystem(x, np.ones(len(x), np.int32), tag, np.zeros(3), np.full(3, 48.0), [0], O.rc2(), 0.0, shuffle_seed=2)
+    keep = np.concatenate([np.arange(min(ball, 3)), np.arange(ball, len(x))]).astype(np.int32)
+    rows = [S.nbr[S.nbr_off[i]:S.nbr_off[i + 1]] for i in keep]
+    S.ilist, S.inum, S.nbr = keep, len(keep), np.concatenate(rows).astype(np.int32)
+    S.nbr_off = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    assert len(S.nbr) <= 80 * S.inum
+    if ball:
+        near = np.linalg.norm(S.x[rows[0]] - S.x[0], axis=1) < 4.0
+        assert near.sum() == ball - 1 and (S.tag[rows[0][near]] > 1).all()
+    trips, quads = O.build_lists(S)
+    assert len(trips) > 50 and (len(quads) > 0) == (orders[2] > 0)
+    model = GpuModel(pf)
+    P = LmpPair(model, {1: W.MASS["C"]})
+    P.build_mb_neighlists(S.x, S.tag, S.ilist, S.numneigh, S.nbr_off, S.nbr, skin=0.0)
+    g3, g4 = P.mb_lists()
+    assert np.array_equal(g3, trips) and np.array_equal(g4, quads), (len(trips), len(quads))
+    P.close()
+    model.close()
+
+
 @pytest.mark.parametrize("natoms", [2, 64, 65, 66, 129, 300])
 def test_pair_rows(tmp_path, natoms):
     """1-/2-body forces and every tally of owners with up to natoms - 1
