@@ -336,11 +336,14 @@ struct fx_table {
         if (atom < 0) return;
         unsigned h = ((unsigned)atom * 2654435761u) >> 8;
         int s = (int)(h & (CAP - 1));
-        bool found = false;
-        for (int probe = 0; probe < 16; probe++) {
-            const int prev = atomicCAS(&key[s], -1, atom);
-            if (prev == -1 || prev == atom) { found = true; break; }
+        int prev = atomicCAS(&key[s], -1, atom);
+        bool found = prev == -1 || prev == atom;
+        // the further probes in a loop: unrolled they are half of the kernel's code
+#pragma unroll 1
+        for (int probe = 1; probe < 16 && !found; probe++) {
             s = (s + 1) & (CAP - 1);
+            prev = atomicCAS(&key[s], -1, atom);
+            found = prev == -1 || prev == atom;
         }
         if (!found) {
             for (int k = 0; k < 3; k++) fx_atomic(acc + (long)CHX_FACC_STRIDE * atom + 2 * k, v[k], bad);

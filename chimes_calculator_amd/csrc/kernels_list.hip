@@ -268,6 +268,11 @@ __device__ __forceinline__ void lane_contract4(const float *__restrict__ img, co
 // across the loop made every kernel here spill (3-body D = 7: 43 registers,
 // 1.64 against 1.43 ms).
 // ---------------------------------------------------------------------------
+// Wavefronts per SIMD.  The targets hold the 3-body kernels for D <= 8 to 128
+// registers and for D <= 11 to 168; at D = 8 and 11 a few spill (32 and 12 bytes
+// of scratch), which costs less than a wavefront: 22 M carbon triplets, D = 8
+// 1.31 ms at four wavefronts, 1.45 at three without scratch; D = 11 2.17 ms at
+// three, 2.54 at two.
 template <int NB, int D>
 constexpr int lane_waves()
 {

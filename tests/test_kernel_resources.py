@@ -56,3 +56,21 @@ def pick(kernels, prefix):
 def test_no_scratch(kernels, prefix):
     for n, k in pick(kernels, prefix).items():
         assert k[".private_segment_fixed_size"] == 0, n
+
+
+@pytest.mark.parametrize("prefix", ["k_lane<", "k_eval2<"])
+def test_scalar_spills(kernels, prefix):
+    """The force table's probes are a loop: unrolled, each kernel that adds to
+    it held the probes' execution masks in spilled scalar registers."""
+    for n, k in pick(kernels, prefix).items():
+        assert k[".sgpr_spill_count"] <= 2, n
+
+
+def test_lane_wavefronts(kernels):
+    """k_lane's registers allow the wavefronts per SIMD it is compiled for
+    (512 registers a lane), with little or no scratch."""
+    for n, k in pick(kernels, "k_lane<").items():
+        nb, D = (int(v) for v in n[n.index("<") + 1:-1].split(","))
+        waves = (4 if D <= 8 else 3 if D <= 11 else 2) if nb == 3 else (3 if D <= 3 else 2)
+        assert 512 // ((k[".vgpr_count"] + 7) // 8 * 8) >= waves, n
+        assert k[".private_segment_fixed_size"] <= (32 if nb == 3 and D in (8, 11) else 0), n
