@@ -1032,7 +1032,12 @@ __global__ __launch_bounds__(64) void k_enum_big(chx_enum_args x)
 // time waiting): in large batches four owners' loads are in flight together
 // (C/O batch of 4096 configurations, 39 M records, beside the 2-body kernel:
 // 345 -> 214 us); small batches keep an owner a wavefront, since they do not
-// fill the device otherwise (1536 water atoms: 6.6 us, 12 with four).
+// fill the device otherwise (1536 water atoms: 6.6 us, 12 with four).  The
+// table has room for 64 / OWN groups; with more, each record's position takes
+// loads of its own, and four owners a wavefront stay the better split: 1500
+// configurations (230,000 atoms), four owners, two and one, us: 9 groups 77,
+// 102, 138; 25 groups (three elements) 110, 107, 137; 36: 111, 133, 147; 72:
+// 115, 131, 150; 360: 101, 110, 130 (only up to 16, 32 and 64 by table).
 template <int OWN>
 __global__ __launch_bounds__(256) void k_place(chx_enum_args x)
 {
