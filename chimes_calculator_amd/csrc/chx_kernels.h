@@ -19,8 +19,6 @@ struct chx_red_model {
     const double *eoff;
 };
 
-__global__ void k_fill_i32(int *p, long n, int v);
-__global__ void k_fill_f64(double *p, long n);
 __global__ void k_prep(int natoms, int ncfg, const int *cfg_atom_off, const chx_cfg *cfgs, const double *pos,
                        const int *types, chx_atom_s *as, chx_atom_n *an, int *cell_count,
                        const int *cfg_item_off, int *in_cfg, int *item_cfg);

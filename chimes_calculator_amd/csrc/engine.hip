@@ -366,7 +366,9 @@ std::vector<float> quad_lane_image(const double *C, int D)
 // own copy for the life of the process; host code uses the address that
 // hipGetSymbolAddress returns for the current device (scratch_init, once per
 // device at engine creation), never the array's name.
-constexpr size_t CHX_SCRATCH_BYTES = (size_t)CHX_STATIC_MAX_CLUSTERS * 416 + 8 * 256;
+// 4-body: six distances, six pair vectors, four types, energy, four force
+// vectors, stress (360 bytes), in six 256-byte aligned parts.
+constexpr size_t CHX_SCRATCH_BYTES = (size_t)CHX_STATIC_MAX_CLUSTERS * 360 + 6 * 256;
 static __device__ __align__(256) char scratch[CHX_SCRATCH_BYTES];
 
 namespace {
@@ -1955,7 +1957,7 @@ int chx_eval_clusters_static(chx_engine *e, chx_model *m, int nb, int n, const d
         const int P = nb * (nb - 1) / 2;
         hipStream_t st = e->st;
         // scratch layout (each part 256-byte aligned): distances, pair vectors,
-        // types, energy, forces, stress, last-term scalars, flags
+        // types, energy, forces, stress
         size_t off = 0;
         auto take = [&](size_t bytes) {
             char *p = base + off;

@@ -72,18 +72,6 @@ __device__ __forceinline__ int find_cfg(const int *off, int n, int r)
     return lo;
 }
 
-__global__ void k_fill_i32(int *p, long n, int v)
-{
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; i < n; i += (long)gridDim.x * blockDim.x) p[i] = v;
-}
-
-__global__ void k_fill_f64(double *p, long n)
-{
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    for (; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // Atom preparation: one thread per replicated atom.
 // ---------------------------------------------------------------------------

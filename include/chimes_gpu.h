@@ -179,7 +179,7 @@ int chimes_gpu_compute_clusters(chimes_gpu_model *m, int nb, int n, const double
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as chimes_gpu_compute_clusters; the clusters'
  * inputs and outputs are staged in a static device array of the library
- * (about 52 MiB, held on each GPU the library runs on until the process
+ * (about 45 MiB, held on each GPU the library runs on until the process
  * ends), so n is at most CHIMES_GPU_STATIC_MAX_CLUSTERS (a larger n is an
  * error) and no call allocates.  All calls on one GPU share that array: calls
  * that overlap on one GPU race. */

@@ -51,3 +51,17 @@ def test_static_entry_matches_allocating_entry(model_dir):
     rc, _, _, _ = call(L, "chimes_gpu_compute_clusters_static", m.h, 4, big, dist, dr, types)
     assert rc != 0 and "out of range" in cc._err()
     m.close()
+
+
+def test_static_entry_at_capacity(model_dir):
+    """The largest call it takes, with the largest clusters."""
+    import chimes_calculator_amd as cc
+    L = cc.lib()
+    m = cc.GpuModel(os.path.join(model_dir, "water_2b3b4b.txt"))
+    n = 131072
+    dist, dr, types = clusters(np.random.default_rng(0xC0DE08), 4, n, 1.0, 4.0, 2)
+    r0, E0, F0, S0 = call(L, "chimes_gpu_compute_clusters", m.h, 4, n, dist, dr, types)
+    r1, E1, F1, S1 = call(L, "chimes_gpu_compute_clusters_static", m.h, 4, n, dist, dr, types)
+    assert r0 == 0 and r1 == 0, cc._err()
+    assert np.array_equal(E0, E1) and np.array_equal(F0, F1) and np.array_equal(S0, S1)
+    m.close()
