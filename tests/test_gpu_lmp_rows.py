@@ -1,7 +1,8 @@
-"""The pair style's list kernel where its bit rows end: owners whose filtered
-rows hold just below, at and above 64 and 256 candidates (word and working-set
-edges, the large form included), list entries compared exactly with the
-oracle's."""
+"""The pair style's list kernels where their bit rows end: owners whose filtered
+rows hold just below, at and above 64 and 256 candidates and the most of 512
+(word and working-set edges, the large form included), in both forms, list
+entries compared exactly with the oracle's.  Candidate counts and row lengths
+are asserted."""
 import numpy as np
 import pytest
 
@@ -12,23 +13,34 @@ from oracle_bindings import LmpOracle
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("natoms,rc4", [(2, 3.5), (64, 3.5), (65, 3.5), (66, 0.9), (129, 2.0), (257, 1.2), (259, 1.2)])
-def test_rows(tmp_path, natoms, rc4):
+@pytest.mark.parametrize("natoms,rc4,shell", [
+    (2, 3.5, 0), (64, 3.5, 0), (65, 3.5, 0), (66, 0.9, 0),  # one wavefront per owner, up to 64 candidates
+    (2, 3.5, 90), (64, 3.5, 90), (65, 3.5, 90), (66, 0.9, 90),  # the row-wise form: 63, 64, 65 candidates
+    (129, 2.0, 0), (257, 1.2, 0), (258, 1.2, 0), (259, 1.2, 0), (513, 0.8, 0),
+])
+def test_rows(tmp_path, natoms, rc4, shell):
     from chimes_calculator_amd import GpuModel, LmpPair
-    # natoms atoms in a ball of 2.2 A: the owner of the lowest tag has all others in its row
+    # natoms atoms in a ball of 2.2 A about the one of the lowest tag, which so
+    # has natoms - 1 candidates; shell: atoms that lengthen its row beyond the
+    # many-body cutoffs
     m = W.Model("ball", ["C"], (4, 3, 3), (5.0, 4.0, rc4), {frozenset(("C",)): 0.05}, seed=natoms)
     pf = m.write(str(tmp_path / "ball.txt"))
     rng = np.random.default_rng(natoms)
-    v = rng.normal(size=(natoms, 3))
-    x = 10.0 + v / np.linalg.norm(v, axis=1)[:, None] * 2.2 * rng.random((natoms, 1)) ** (1.0 / 3.0)
+    v = rng.normal(size=(natoms + shell, 3))
+    r = np.where(np.arange(natoms + shell) < natoms, 2.2 * rng.random(natoms + shell) ** (1.0 / 3.0), 4.5)
+    r[0] = 0.0
+    x = 10.0 + v / np.linalg.norm(v, axis=1)[:, None] * r[:, None]
+    tag = np.concatenate([[1], rng.permutation(natoms + shell - 1) + 2]).astype(np.int32)
     O = LmpOracle(pf)
-    S = LmpSystem(x, np.ones(natoms, np.int32), rng.permutation(natoms).astype(np.int32) + 1, np.zeros(3),
-                  np.full(3, 20.0), [0], O.rc2(), 0.0, shuffle_seed=1)
-    keep = 3 if natoms > 100 else natoms  # owners: the lists of a few low tags are long enough
+    S = LmpSystem(x, np.ones(len(x), np.int32), tag, np.zeros(3), np.full(3, 20.0), [0], O.rc2(), 0.0, shuffle_seed=1)
+    keep = 1 if shell else 3 if natoms > 100 else natoms  # owners: the lists of a few low tags are long enough
     S.ilist = np.argsort(S.tag[: S.nlocal])[:keep].astype(np.int32)
     rows = [S.nbr[S.nbr_off[i]:S.nbr_off[i + 1]] for i in S.ilist]
     S.inum, S.nbr = keep, np.concatenate(rows).astype(np.int32)
     S.nbr_off = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    near = np.linalg.norm(S.x[rows[0]] - S.x[S.ilist[0]], axis=1) < 4.0
+    assert near.sum() == natoms - 1 and len(rows[0]) == natoms + shell - 1
+    assert (len(S.nbr) > 80 * S.inum) == (shell > 0 or natoms > 100)
     trips, quads = O.build_lists(S)
     model = GpuModel(pf)
     P = LmpPair(model, {1: W.MASS["C"]})

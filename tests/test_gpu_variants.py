@@ -1,11 +1,11 @@
 """Every 3-/4-body kernel variant the autotuner can choose, pinned to the
 reference's goldens.
 
-The variants are the matrix-core kernels with 64- and 32-cluster tiles, the
-vector-unit kernel, and the one-cluster-per-lane kernel with the 3-body
-contraction on the matrix cores (FP32-mixed, D <= 10; the 4-body matrix-core
-kernels cover D <= 4; outside those ranges the request runs on the vector
-units).  Each is forced in turn through
+The variants are the matrix-core kernels with 64- and 32-cluster tiles (the
+4-body ones cover D <= 4; outside that the request runs with one cluster per
+lane) and the one-cluster-per-lane kernels, which two numbers name: FP64 on the
+vector units, FP32-mixed with the contraction on the matrix cores (4-body
+D <= 4).  Each is forced in turn through
 chimes_gpu_set_variants and evaluated in FP64 and FP32-mixed on:
   * the dense-dimension scan (tests/golden/dscan_cases.json): two-type C/O
     models covering every instantiated dense dimension, 3-body D = 2..13
