@@ -154,7 +154,11 @@ __global__ void k_cell_fill(int natoms, const chx_atom_n *__restrict__ an, const
 // + 5.8 + 2.2 us and three gaps against 5.3 us; a calculator call of 64 atoms
 // 155 -> 142 us, a plan of 729 carbon atoms 144 -> 132 us).  Up to
 // CHX_SETUP_ATOMS atoms, one a thread, and as many cells and words to clear as
-// one workgroup passes over in a few microseconds.
+// one workgroup passes over in a few microseconds.  C/O plans, this kernel
+// against the four launches, us: 2 atoms 98 and 113, 256: 102 and 115, 512:
+// 110 and 121, 1024: 127 and 138; 26 configurations of 8 atoms (the most words
+// to clear, 32,000) 107 and 119; and at the least favourable end 600 atoms over
+// 3375 cells 107 and 113, 900 atoms over them 109 and 109.
 __global__ __launch_bounds__(1024) void k_setup_small(chx_setup_args x)
 {
     __shared__ int cnt[CHX_SETUP_CELLS];

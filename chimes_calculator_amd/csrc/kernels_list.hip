@@ -473,7 +473,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NB == 4 && 
 
 // Tiles per wavefront of the lane kernels: four where that leaves 4096
 // workgroups (four for each of the 1024 the device holds at once), else one,
-// so that a short list still reaches every compute unit.
+// so that a short list still reaches every compute unit.  One, two and four
+// tiles, us: 1.3 M slots (C/O 4-body) 145, 129, 129; 2.1 M 227, 205, 208;
+// 4.7 M (C/O 3-body) 295, 281, 281; 5.1 M (C/O 4-body) 530, 472, 436; but 0.2 M
+// 25, 28, 35, and 0.4 to 0.8 M 52, 58, 63 and 100, 94, 108.  Two or four tiles
+// from 1.3 M slots would be 3-18% shorter than the one that the line gives
+// lists up to 4.2 M.
 constexpr long LANE_TILES = 4;
 
 void launch_evalv(int nb, int D, int prec, const chx_list_args &la, hipStream_t st)

@@ -1,8 +1,8 @@
 // LAMMPS pair style chimesFF (etc/lmp/src/pair_chimes.cpp) on the GPU, one
 // process's local and ghost atoms per call:
 //   k_lmp_pair      1- and 2-body loops of PairCHIMES::compute (567-656)
-//   k_lmp_lists     PairCHIMES::build_mb_neighlists (321-478)
-//   k_lmp_clusters  3- and 4-body loops (673-829) over those lists
+//   k_lmp_lists, k_lmp_lists_short  PairCHIMES::build_mb_neighlists (321-478)
+//   k_lmp_near, k_lmp_clusters      3- and 4-body loops (673-829) over those lists
 //   k_lmp_out       fixed-point accumulators -> forces and tallies
 // Every tally of Pair::ev_tally_mb (etc/lmp/etc/pair.cpp:1425-1482) is added
 // in the exact fixed-point form of the batch pipeline, so results do not
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(64) void k_lmp_lists_short(chx_lmp_args A, double p
 // as the reference forms them (ij, ik, jk / ij, ik, il, jk, jl, kl; x_b - x_a),
 // the terms of compute_3B / compute_4B, then the forces of every member and
 // the tallies of ev_tally_mb (energy and virial shared equally by the
-// members; the global part kept per owner atom).
+// members; the global part in CHX_LMP_GSLOTS copies).
 // ---------------------------------------------------------------------------
 // compute_3B_tab (chimesFF.cpp:2183-2313): exclusion and the cutoffs of the
 // mapped slots as compute_3B, then the table at the runtime pair distances
