@@ -38,7 +38,9 @@ __device__ __forceinline__ void cheby(double r, const chx_slot &s, R (&T)[D], R 
     dT[0] = (R)0;
     if constexpr (sizeof(R) == 8) {
         // V_i = U_i dx/dr by the same recurrence, so dT_i/dr = i V_{i-1}; one
-        // fused operation a step
+        // fused operation a step.  Rms error of dT_i/dr against 113-bit values,
+        // this form and the one rounded step by step below: D = 4 3.588e-16 and
+        // 3.592e-16, D = 8 1.41e-15 and 1.43e-15, D = 13 3.66e-15 and 3.69e-15
         R V[D];
         V[0] = dxdr;
         if (D > 1) V[1] = two_x * dxdr;
